@@ -118,10 +118,14 @@ struct GemvParams {
     uint32_t m, k, n, ldo;
 };
 bool launch_gemv(const GemvParams& p, hipStream_t stream);
+// up to three weights over the same rows: one GEMM where they allow it (same a,
+// m, k, type, accumulate; shapes the DMA GEMM takes), else one after the other.
+// split: the DMA GEMM's operand images of a (gemm_split_image) are written
+bool launch_gemvs(const GemvParams* ps, int count, bool split, hipStream_t stream);
 
-// the k or v projection of a prefill with attentionMixer's per-token work
-// as its epilogue: QK-RMSNorm (gamma), rotate-half RoPE (freqs), then the
-// row appended to the bf16 cache and to the flash kernel's fp16 copy
+// attentionMixer's per-token work after a prefill's k or v projection:
+// QK-RMSNorm (gamma), rotate-half RoPE (freqs), then the row appended to the
+// bf16 cache and to the flash kernel's fp16 copy
 struct KvEpilogue {
     uint16_t* cache;      // bf16 [kvHeads][capacity][dim]
     void* work;           // fp16 [kvHeads][T][dim]
@@ -132,7 +136,6 @@ struct KvEpilogue {
     uint64_t capacity;
     uint32_t* rangeFlag;  // as PrefillParams::rangeFlag
 };
-bool launch_gemm_kv(const GemvParams& p, const KvEpilogue& e, hipStream_t stream);
 // whether launch_gemv splits p.a into the bf16 images a following
 // launch_gemm_kv_pair can reuse (aSplit)
 bool gemm_splits_a(const GemvParams& p);
@@ -142,9 +145,8 @@ uint16_t* gemm_split_image(const GemvParams& p);
 // launch_gemv for a p that takes the DMA GEMM, with gemm_split_image(p)
 // already written (p.a is not read)
 bool launch_gemv_presplit(const GemvParams& p, hipStream_t stream);
-// the k and v projections of the same rows: one GEMM over both weights, then
-// the epilogue as its own kernel, where the shapes allow; otherwise two
-// launch_gemm_kv calls
+// the k and v projections of the same rows (one GEMM over both weights where
+// the shapes allow), then the epilogue as its own kernel
 // fold: also write prep's cos/sin table (rope, may be null) and zero the
 // working copies' pad rows; *folded says whether that was done
 bool launch_gemm_kv_pair(const GemvParams& pk, const GemvParams& pv, const KvEpilogue& ek, const KvEpilogue& ev,

@@ -13,8 +13,8 @@
 // (4, 8, 16 or 32 weights), one wave owns GEMV_ROWS weight rows and keeps an
 // fp32 accumulator per (weight row, a row), and a shuffle tree reduces the
 // lanes. Up to GEMM_MIN_M - 1 rows of a run as blocks of 8 along grid.y;
-// more rows take gemm_kernel on MFMA, and bf16 weights with enough rows for
-// 256 x 256 tiles split_a_kernel and gemm_dma_kernel.
+// more rows take split_a_kernel and gemm_dma_kernel on MFMA, or gemm_kernel
+// where k is not whole 32-wide steps (128 for Q8 and Q4).
 #include <type_traits>
 #include "context.hpp"
 #include "device.hpp"
@@ -95,7 +95,8 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
 }
 
 /*
-    gemm_kernel: many rows of a (prefill), on v_mfma_f32_16x16x32_bf16.
+    gemm_kernel: many rows of a (prefill), on v_mfma_f32_16x16x32_bf16, for
+    the shapes gemm_dma_kernel does not take.
     A stays fp32 at the boundary; each value is split into a bf16 high part
     and the bf16 residual, and hi.B + lo.B keeps about 16 bits of it. BF16
     weights and the Q8/Q4 codes are exact in bf16; fp32 weights are split
@@ -109,18 +110,11 @@ __global__ __launch_bounds__(256) void gemv_kernel(GemvParams p) {
 */
 constexpr int GM_BM = 128, GM_BN = 128, GM_BK = 32, GM_AS = GM_BK + 8;
 constexpr int GM_OP = GM_BM * GM_AS;   // bf16 elements of one operand buffer
-constexpr int GM_ES = GM_BN + 4;       // row stride (floats) of the epilogue's half tile
 
-/* KV: the k / v epilogue of a prefill (launch_gemm_kv) instead of the plain
-   store. It takes the tile through LDS in two halves of 64 rows; four threads
-   per row, each 32 consecutive columns, which lie in one head (dim 64 or 128,
-   tiles start on multiples of 128). */
-template <int TYPE, bool KV>
-__global__ __launch_bounds__(256) void gemm_kernel(GemvParams p, KvEpilogue ep, uint32_t kSlice) {
+template <int TYPE>
+__global__ __launch_bounds__(256) void gemm_kernel(GemvParams p, uint32_t kSlice) {
     constexpr bool SPLIT_W = TYPE == 0, QUANT = TYPE >= 2;
-    constexpr int OPS = (SPLIT_W ? 4 : 3) * GM_OP;   // Ah, Al, Bh (, Bl)
-    constexpr int EPI = KV ? 64 * GM_ES * 2 : 0;      // the half tile in fp32, counted in bf16
-    __shared__ __align__(16) __bf16 smem[OPS > EPI ? OPS : EPI];
+    __shared__ __align__(16) __bf16 smem[(SPLIT_W ? 4 : 3) * GM_OP];   // Ah, Al, Bh (, Bl)
     __bf16* const Ah = smem;
     __bf16* const Al = smem + GM_OP;
     __bf16* const Bh = smem + 2 * GM_OP;
@@ -274,126 +268,56 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemvParams p, KvEpilogue ep, 
             }
     }
     // the accumulator layout: lane holds rows 4 (lane / 16) + r of column lane % 16
-    if constexpr (!KV) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t n = n0 + 64 * wn + 16 * j + (lane & 15);
-                if (n >= N) continue;
-                const float b = p.bias ? p.bias[n] : 0.0f;
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t n = n0 + 64 * wn + 16 * j + (lane & 15);
+            if (n >= N) continue;
+            const float b = p.bias ? p.bias[n] : 0.0f;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t m = m0 + 64 * wm + 16 * i + 4 * (lane >> 4) + r;
-                    if (m >= M) continue;
-                    // a K slice writes its own partial tile (no bias, no accumulate)
-                    float* o = p.out + size_t(blockIdx.z) * M * p.ldo + size_t(m) * p.ldo + n;
-                    *o = (p.accumulate ? *o : 0.0f) + acc[i][j][r] + b;
-                }
-            }
-    } else {
-        float* tile = reinterpret_cast<float*>(smem);
-        const uint32_t D = ep.dim;
-        const int row = tid >> 2, c0 = 32 * (tid & 3);   // half-tile row, first column
-        const uint32_t n = n0 + uint32_t(c0);                // k or v column: head n / D, dim n % D
-        const uint32_t d0 = n % D, head = n / D, hc = uint32_t(c0) - d0;
-        const uint32_t half = ep.freqs ? ep.rot / 2 : 0;
-        bool bad = false;   // an fp16 conversion out of range
-        for (int hf = 0; hf < 2; ++hf) {
-            __syncthreads();   // the operand reads, or the previous half's tile reads, are done
-            if (wm == hf) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const uint32_t c = 64 * wn + 16 * j + (lane & 15);
-                        const float b = p.bias && n0 + c < N ? p.bias[n0 + c] : 0.0f;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) tile[(16 * i + 4 * (lane >> 4) + r) * GM_ES + c] = acc[i][j][r] + b;
-                    }
-            }
-            __syncthreads();
-            const float* tr = tile + row * GM_ES;
-            float x[32];
-#pragma unroll
-            for (int e = 0; e < 32; e += 4) {
-                const floatx4 t = *reinterpret_cast<const floatx4*>(tr + c0 + e);
-                x[e] = t[0];
-                x[e + 1] = t[1];
-                x[e + 2] = t[2];
-                x[e + 3] = t[3];
-            }
-            // the head's D / 32 threads are lanes 4 t + (0..3) or (0, 1) / (2, 3): the
-            // butterflies run in every lane, rows past M or columns past N included
-            float inv = 1.0f;
-            if (ep.gamma) {   // rmsNormRow (LocalModel.hpp:1341-1348)
-                float ss = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 32; ++e) ss = fmaf(x[e], x[e], ss);
-                ss += __shfl_xor(ss, 1, WAVE);
-                if (D == 128) ss += __shfl_xor(ss, 2, WAVE);
-                inv = 1.0f / sqrtf(ss / float(D) + ep.eps);
-            }
-            const uint32_t m = m0 + 64 * hf + row;
-            if (m < M && n < N) {
-                const uint32_t pos = ep.start + m;
-                float y[32];
-#pragma unroll
-                for (int e = 0; e < 32; ++e) y[e] = ep.gamma ? x[e] * inv * (ep.gamma[d0 + e] + ep.offset) : x[e];
-                if (half) {   // rotate-half pairs (LocalModel.hpp:2624-2641), the angle float(pos) * freq
-                    const float fpos = float(pos);
-#pragma unroll
-                    for (int e = 0; e < 32; ++e) {
-                        const uint32_t d = d0 + e;
-                        if (d < 2 * half) {
-                            const bool low = d < half;
-                            const uint32_t dp = low ? d + half : d - half;
-                            const float xp = ep.gamma ? tr[hc + dp] * inv * (ep.gamma[dp] + ep.offset) : tr[hc + dp];
-                            float sn, cs;
-                            sincosf(fpos * ep.freqs[low ? d : dp], &sn, &cs);
-                            y[e] = low ? y[e] * cs - xp * sn : y[e] * cs + xp * sn;
-                        }
-                    }
-                }
-                uint16_t* cdst = ep.cache + (size_t(head) * ep.capacity + pos) * D + d0;
-                _Float16* wdst = static_cast<_Float16*>(ep.work) + (size_t(head) * ep.T + pos) * D + d0;
-#pragma unroll
-                for (int e = 0; e < 32; e += 8) {
-                    u32x4 wb;
-                    half8 wh;
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                        wb[t] = uint32_t(float_to_bf16_bits(y[e + 2 * t])) |
-                                (uint32_t(float_to_bf16_bits(y[e + 2 * t + 1])) << 16);
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) wh[t] = to_f16_checked(y[e + t], bad);
-                    *reinterpret_cast<u32x4*>(cdst + e) = wb;
-                    *reinterpret_cast<half8*>(wdst + e) = wh;
-                }
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t m = m0 + 64 * wm + 16 * i + 4 * (lane >> 4) + r;
+                if (m >= M) continue;
+                // a K slice writes its own partial tile (no bias, no accumulate)
+                float* o = p.out + size_t(blockIdx.z) * M * p.ldo + size_t(m) * p.ldo + n;
+                *o = (p.accumulate ? *o : 0.0f) + acc[i][j][r] + b;
             }
         }
-        raise_range_flag(ep.rangeFlag, bad);
-    }
 }
 
 /*
-    gemm_dma_kernel: bf16 weights and enough rows for 256 x 256 tiles, after
-    split_a_kernel has split a into bf16 high parts and residuals ([M][K]
-    each). Four waves of 128 x 128 (8 x 8 v_mfma_f32_16x16x32_bf16 tiles, the
-    256 fp32 accumulators per lane in AGPRs, one workgroup per CU); per
-    32-wide K step a wave reads 24 KB of operands from LDS for 128 MFMAs.
-    Every operand comes in by DMA (global_load_lds, 1 KB blocks) into a
-    three-stage LDS ring of 48 KB stages, step t + 2 issued between step t's
-    MFMAs, so nothing passes through registers or the VALU and each step's
-    loads have two steps of compute to land; one barrier per step. Within a
-    1 KB block (16 rows of 64 bytes) row r keeps its 16-byte chunk c at
-    position c ^ s(r % 16), s(x) = ((x / 2) % 4) ^ (x / 8): the 16 rows of an
-    operand read fall on distinct banks both as one 256-byte access and as
-    two 128-byte halves.
+    gemm_dma_kernel: the MFMA GEMM of every aligned shape (K whole steps of
+    32; whole groups of four for Q8 and Q4), after split_a_kernel has split a
+    into bf16 high parts and residuals ([M][K] each). Every operand comes in
+    by DMA (global_load_lds, 1 KB blocks) into a three-stage LDS ring, step
+    t + 2 issued between step t's MFMAs, so nothing passes through registers
+    or the VALU on its way in and each step's loads have two steps of compute
+    to land; one barrier per step. 2 x WN waves of BM/2 x BN/WN outputs, two
+    waves on a SIMD wherever the tile allows, so that one's operand reads
+    after the barrier hide behind the other's MFMAs (256 x 256 tiles: 450 us
+    with eight waves, 453 with four at 8192 x 4096 -> 4096, 170 and 187 on a
+    cool chip at 500 rows; reading the next step's operands before the last
+    row tile instead measured 20% slower). It is bound by the MFMA rate at the
+    clock the chip holds: 1999 x 4096 -> 4096 in bf16, 128 x 256 tiles, 127 us
+    (gemm_kernel, which splits a in registers and stores it to LDS behind two
+    barriers a step: 190); Q8 500 x 4096 -> 12288 137 us (217).
+      BF16  up to 256 x 256 tiles
+      F32   w in fp32 in LDS, split on its way into the operand registers
+            (a third product, hi_a.lo_w)
+      Q8/Q4 the codes in LDS as stored, widened to bf16 (exactly) on their
+            way into the operand registers; one 32-wide step is one scale
+            block: its products go through a scratch accumulator and are
+            added in times the column's scale. The scales come in by DMA too,
+            four steps at a time.
+    In LDS, a 1 KB block of bf16 is 16 rows of 64 bytes; row r keeps its
+    16-byte chunk c at position c ^ s(r % 16), s(x) = ((x / 2) % 4) ^ (x / 8):
+    the 16 rows of an operand read fall on distinct banks both as one
+    256-byte access and as two 128-byte halves. A block of fp32 is 8 rows of
+    128 bytes, chunk c at c ^ ((r / 2) % 8), for the same reason; Q8 (32 rows
+    of 32 bytes) and Q4 (64 rows of 16) need no swizzle.
 */
-constexpr int GD_BM = 256, GD_BN = 256, GD_BK = 32, GD_STAGES = 3;
-constexpr int GD_OPB = GD_BM * GD_BK * 2;   // bytes of one operand's tile per step (16 KB)
-constexpr int GD_STAGE = 3 * GD_OPB;         // a hi, a lo, w
+constexpr int GD_BK = 32, GD_STAGES = 3;
 
 __global__ __launch_bounds__(256) void split_a_kernel(const float* a, bf16x8* hi, bf16x8* lo, uint64_t pieces) {
     for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < pieces; i += uint64_t(gridDim.x) * 256) {
@@ -419,114 +343,253 @@ __device__ __forceinline__ void gd_wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
 }
 
-/* w2: columns from nSplit on come from w2's rows (n - nSplit), a multiple of
-   256 so that no tile straddles the two; null for one weight */
-__global__ __launch_bounds__(256) void gemm_dma_kernel(GemvParams p, const __bf16* ahi, const __bf16* alo,
-                                                       const void* w2, uint32_t nSplit) {
-    __shared__ __align__(16) uint8_t smem[GD_STAGES * GD_STAGE];
-    const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) >> 1, wn = (tid >> 6) & 1;
+/* up to three weights over the same rows of a share a launch: segment s has
+   the tile columns from `start` (in columns, a multiple of the tile's) on */
+constexpr int GD_SEGS = 3;
+struct GemmSeg {
+    const void* w;
+    const float *scales, *bias;
+    float* out;
+    uint32_t n, ldo, start;
+};
+struct GemmArgs {
+    const __bf16 *ahi, *alo;
+    GemmSeg seg[GD_SEGS];
+    uint32_t nseg, m, k, accumulate;
+    uint32_t columns;      // of all segments, each padded to whole tiles
+    uint32_t sliceSteps;   // K steps per slice (blockIdx.y)
+    float* part;           // with K slices: their partial tiles, [slice][m][columns]
+};
+
+__device__ __forceinline__ int segment_of(const GemmArgs& a, uint32_t n) {
+    int s = 0;
+#pragma unroll
+    for (int i = 1; i < GD_SEGS; ++i)
+        if (uint32_t(i) < a.nseg && n >= a.seg[i].start) s = i;
+    return s;
+}
+
+template <int TYPE> constexpr int gd_row_bytes() { return TYPE == 0 ? 128 : (TYPE == 1 ? 64 : (TYPE == 2 ? 32 : 16)); }
+template <int TYPE, int BM, int BN> constexpr int gd_stage() { return 2 * BM * 64 + BN * gd_row_bytes<TYPE>(); }
+/* eight Q8 codes to bf16, exactly */
+__device__ __forceinline__ bf16x8 widen_q8(u32x2 c) {
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = __bf16(float(int32_t(c[e / 4] << (24 - 8 * (e % 4))) >> 24));
+    return r;
+}
+/* the low nibbles of eight bytes, less 8, to bf16, exactly */
+__device__ __forceinline__ bf16x8 widen_q4(u32x2 c) {
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = __bf16(float((c[e / 4] >> (8 * (e % 4))) & 0xFu) - 8.0f);
+    return r;
+}
+
+template <int TYPE, int BM, int BN, int WN>
+__global__ __launch_bounds__(128 * WN, 2) void gemm_dma_kernel(GemmArgs a) {
+    constexpr bool QUANT = TYPE >= 2;
+    constexpr int W = 2 * WN;                           // waves, 2 x WN
+    constexpr int TI = BM / 32, TJ = BN / WN / 16;     // 16 x 16 tiles of a wave's BM/2 x BN/WN
+    constexpr int AOP = BM * 64;                        // bytes of one image of a per step
+    constexpr int RB = gd_row_bytes<TYPE>();            // bytes of a w row per step
+    constexpr int BROWS = 1024 / RB;                    // w rows per DMA block
+    constexpr int STAGE = gd_stage<TYPE, BM, BN>();
+    constexpr int AJ = BM / 16 / W;                       // DMA blocks of one image of a per wave and step
+    constexpr int BJ = BN / BROWS >= W ? BN / BROWS / W : 1;   // of w (fewer blocks than waves: some are loaded twice)
+    constexpr int NB = 2 * AJ + BJ;
+    __shared__ __align__(16) uint8_t smem[GD_STAGES * STAGE + (QUANT ? 2 * BN * 16 : 0)];
+    const int tid = threadIdx.x, lane = tid & 63, wm = (tid >> 6) / WN, wn = (tid >> 6) % WN;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: DMA targets are scalar
-    const uint32_t K = p.k, M = p.m, N = p.n;
-    const uint32_t ntN = (N + GD_BN - 1) / GD_BN;
+    const uint32_t K = a.k, M = a.m;
+    const uint32_t ntM = (M + BM - 1) / BM, ntN = a.columns / BN;
     // consecutive workgroups go to different XCDs: remap them so that each XCD
-    // takes a band of whole rows of tiles (its L2 then holds a band of a and
-    // every XCD reads w), when the tile count splits evenly over the eight
+    // takes a run of tiles, when they split evenly over the eight; runs go
+    // down four tile rows before the next tile column, so that the tiles an
+    // XCD holds at once share both their rows of a and their rows of w in its L2
     uint32_t lg = blockIdx.x;
     if (gridDim.x % 8 == 0) lg = (lg % 8) * (gridDim.x / 8) + lg / 8;
-    const uint32_t m0 = (lg / ntN) * GD_BM, n0 = (lg % ntN) * GD_BN;
+    const uint32_t band = lg / (4 * ntN), inBand = lg % (4 * ntN);
+    const uint32_t bandRows = ntM - 4 * band < 4 ? ntM - 4 * band : 4;
+    const uint32_t m0 = (4 * band + inBand % bandRows) * BM, n0 = (inBand / bandRows) * BN;
     const uint32_t ldsBase = lds_address(smem);
+    const uint32_t kBegin = blockIdx.y * a.sliceSteps;
+    const uint32_t kSteps = K / GD_BK - kBegin < a.sliceSteps ? K / GD_BK - kBegin : a.sliceSteps;
 
-    // this wave's twelve DMA blocks of a step: block j is operand j / 4 (a hi,
-    // a lo, w), rows 16 (4 w + j % 4) .. + 15 of its tile; lane l takes row
-    // + l / 4, LDS chunk l % 4, which holds the row's chunk (l % 4) ^ s(l / 4).
-    // Rows past M or N read the last row: they only reach outputs past M or
-    // N, which are not stored.
-    const bool second = w2 && n0 >= nSplit;
-    const uint32_t wn0 = second ? n0 - nSplit : n0, wlim = w2 ? (second ? N - nSplit : nSplit) : N;
-    uint32_t doff[12];
+    // this wave's DMA blocks of a step. Rows past M or N read the last row:
+    // they only reach outputs past M or N, which are not stored.
+    const GemmSeg& S = a.seg[segment_of(a, n0)];
+    const uint32_t wn0 = n0 - S.start;
+    const uint8_t* const wBase = static_cast<const uint8_t*>(S.w) + size_t(kBegin) * RB;
+    const uint8_t* const hiBase = reinterpret_cast<const uint8_t*>(a.ahi) + size_t(kBegin) * 64;
+    const uint8_t* const loBase = reinterpret_cast<const uint8_t*>(a.alo) + size_t(kBegin) * 64;
+    const uint32_t rowStride = K / GD_BK * RB;          // bytes of a w row
+    uint32_t aoff[AJ], woff[BJ];
 #pragma unroll
-    for (int j = 0; j < 12; ++j) {
-        const uint32_t row = 16u * (4u * uint32_t(w) + (j & 3)) + uint32_t(lane >> 2);
+    for (int j = 0; j < AJ; ++j) {   // lane l: row l / 4, LDS chunk l % 4, which holds chunk (l % 4) ^ s(l / 4)
+        const uint32_t row = m0 + 16u * (AJ * uint32_t(w) + j) + uint32_t(lane >> 2);
         const uint32_t chunk = uint32_t(lane & 3) ^ uint32_t(((lane >> 3) & 3) ^ (lane >> 5));
-        const uint32_t g = (j < 8 ? m0 : wn0) + row, lim = j < 8 ? M : wlim;
-        doff[j] = ((g < lim ? g : lim - 1) * K + 8 * chunk) * 2;
+        aoff[j] = ((row < M ? row : M - 1) * K + 8 * chunk) * 2;
     }
-    const uint8_t* const bases[3] = {reinterpret_cast<const uint8_t*>(ahi), reinterpret_cast<const uint8_t*>(alo),
-                                     static_cast<const uint8_t*>(second ? w2 : p.w)};
-    auto dma = [&](uint32_t kt, int j) __attribute__((always_inline)) {
-        const uint32_t stage = kt % GD_STAGES;
-        dma_block(bases[j >> 2] + size_t(kt) * GD_BK * 2, doff[j],
-                  ldsBase + stage * GD_STAGE + (j >> 2) * GD_OPB + (4 * w + (j & 3)) * 1024);
+    const uint32_t wblk = BN / BROWS >= W ? uint32_t(BJ) * w : uint32_t(w) % (BN / BROWS);
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) {
+        constexpr int CPR = RB / 16;   // 16-byte chunks per row
+        const uint32_t r = uint32_t(lane) / CPR, c = uint32_t(lane) % CPR;
+        const uint32_t chunk = TYPE == 0 ? c ^ ((r >> 1) & 3) ^ (4 * ((wblk + j) & 1)) : (TYPE == 1 ? c ^ (((r >> 1) & 3) ^ (r >> 3)) : c);
+        const uint32_t row = wn0 + (wblk + j) * BROWS + r;
+        woff[j] = (row < S.n ? row : S.n - 1) * rowStride + 16 * chunk;
+    }
+    uint32_t soff = 0;
+    const uint8_t* sBase = nullptr;
+    constexpr int SB = BN / 64;   // DMA blocks of four steps' scales: 64 rows each
+    const uint32_t scaleLds = ldsBase + GD_STAGES * STAGE + (w % SB) * 1024;
+    if constexpr (QUANT) {
+        const uint32_t row = wn0 + 64 * (w % SB) + lane;
+        soff = (row < S.n ? row : S.n - 1) * (K / 8);   // K / 32 floats per row
+        sBase = reinterpret_cast<const uint8_t*>(S.scales) + size_t(kBegin) * 4;
+    }
+    auto dma = [&](uint32_t kt, int j) __attribute__((always_inline)) {   // block j of step kt
+        const uint32_t stage = ldsBase + (kt % GD_STAGES) * STAGE;
+        if (j < AJ) dma_block(hiBase + size_t(kt) * 64, aoff[j], stage + (AJ * w + j) * 1024);
+        else if (j < 2 * AJ) dma_block(loBase + size_t(kt) * 64, aoff[j - AJ], stage + AOP + (AJ * w + j - AJ) * 1024);
+        else dma_block(wBase + size_t(kt) * RB, woff[j - 2 * AJ], stage + 2 * AOP + (wblk + j - 2 * AJ) * 1024);
+    };
+    auto dma_scales = [&](uint32_t group) __attribute__((always_inline)) {   // four steps' scales: [BN rows][4]
+        dma_block(sBase + size_t(group) * 16, soff, scaleLds + (group & 1) * (BN * 16));
     };
 
-    floatx4 acc[8][8];
+    floatx4 acc[TI][TJ];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int fr = lane & 15, sw = 16 * ((lane >> 4) ^ ((fr >> 1) & 3) ^ (fr >> 3));   // swizzled chunk of k 8 (lane / 16) ..
-    const uint32_t nk = K / GD_BK;
+        for (int j = 0; j < TJ; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int g = lane >> 4, fr = lane & 15, sw = 16 * (g ^ ((fr >> 1) & 3) ^ (fr >> 3));   // swizzled chunk of k 8 g ..
+    if constexpr (QUANT) dma_scales(0);
 #pragma unroll
-    for (int j = 0; j < 12; ++j) dma(0, j);
-    if (nk > 1) {
+    for (int j = 0; j < NB; ++j) dma(0, j);
+    if (kSteps > 1) {
 #pragma unroll
-        for (int j = 0; j < 12; ++j) dma(1, j);
+        for (int j = 0; j < NB; ++j) dma(1, j);
     }
-    // step kt; MORE: step kt + 2's DMA goes out between its row tiles
+    // step kt; MORE: step kt + 2's DMA goes out between its row tiles, and step
+    // 1 of a group of four also requests the next group's scales (Q8, Q4)
     auto step = [&](uint32_t kt, auto MORE) __attribute__((always_inline)) {
-        // step kt's blocks have landed (in order: step kt + 1's may still be
-        // in flight); after the barrier every wave's have, and every read of
-        // the stage step kt + 2 goes into (that of step kt - 1) is done. Not
-        // __syncthreads(): its fence would wait for step kt + 1's blocks too.
-        if (kt + 1 < nk) gd_wait_vmcnt<12>();
+        constexpr bool more = decltype(MORE)::value;
+        // step kt's blocks have landed (in order: step kt + 1's, and the
+        // scales requested with them, may still be in flight); after the
+        // barrier every wave's have, and every read of the stage step kt + 2
+        // goes into (that of step kt - 1) is done. Not __syncthreads(): its
+        // fence would wait for step kt + 1's blocks too.
+        if (QUANT && kt % 4 == 2 && kt + 2 < kSteps) gd_wait_vmcnt<NB + 1>();
+        else if (kt + 1 < kSteps) gd_wait_vmcnt<NB>();
         else gd_wait_vmcnt<0>();
         lds_barrier();
-        const uint8_t* st = smem + (kt % GD_STAGES) * GD_STAGE;
-        bf16x8 bh[8];
+        const uint8_t* st = smem + (kt % GD_STAGES) * STAGE;
+        if (QUANT && more && kt % 4 == 1 && kt + 3 < kSteps) dma_scales(kt / 4 + 1);
+        const int bw = BN / WN * wn;   // the wave's first column
+        bf16x8 bh[TJ], bl[TYPE == 0 ? TJ : 1];
+        float sc[QUANT ? TJ : 1];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            bh[j] = *reinterpret_cast<const bf16x8*>(st + 2 * GD_OPB + (128 * wn + 16 * j + fr) * 64 + sw);
-        const int ro = (128 * wm + fr) * 64 + sw;
+        for (int j = 0; j < TJ; ++j) {
+            const int row = bw + 16 * j + fr;
+            const uint8_t* br = st + 2 * AOP + row * RB;
+            if constexpr (TYPE == 1) {
+                bh[j] = *reinterpret_cast<const bf16x8*>(br + sw);
+            } else if constexpr (TYPE == 0) {
+                const int x = (row >> 1) & 7;   // chunks 2 g and 2 g + 1
+                const floatx4 x0 = *reinterpret_cast<const floatx4*>(br + 16 * ((2 * g) ^ x));
+                const floatx4 x1 = *reinterpret_cast<const floatx4*>(br + 16 * ((2 * g + 1) ^ x));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    bh[j][e] = __bf16(x0[e]);
+                    bl[j][e] = __bf16(x0[e] - float(bh[j][e]));
+                    bh[j][4 + e] = __bf16(x1[e]);
+                    bl[j][4 + e] = __bf16(x1[e] - float(bh[j][4 + e]));
+                }
+            } else if constexpr (TYPE == 2) {
+                bh[j] = widen_q8(*reinterpret_cast<const u32x2*>(br + 8 * g));
+            } else {   // byte t of a block: code t low, code t + 16 high
+                const u32x2 c = *reinterpret_cast<const u32x2*>(br + 8 * (g & 1));
+                bh[j] = widen_q4(u32x2{c[0] >> (4 * (g >> 1)), c[1] >> (4 * (g >> 1))});
+            }
+            if constexpr (QUANT)
+                sc[j] = *reinterpret_cast<const float*>(smem + GD_STAGES * STAGE + ((kt / 4) & 1) * (BN * 16) + row * 16 + 4 * (kt % 4));
+        }
+        const int ro = (BM / 2 * wm + fr) * 64 + sw;
         bf16x8 ah = *reinterpret_cast<const bf16x8*>(st + ro);
-        bf16x8 al = *reinterpret_cast<const bf16x8*>(st + GD_OPB + ro);
+        bf16x8 al = *reinterpret_cast<const bf16x8*>(st + AOP + ro);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {   // row tile i + 1's a operands are read while tile i computes
+        for (int i = 0; i < TI; ++i) {   // row tile i + 1's a operands are read while tile i computes
             bf16x8 nh = ah, nl = al;
-            if (i < 7) {
+            if (i + 1 < TI) {
                 nh = *reinterpret_cast<const bf16x8*>(st + ro + (i + 1) * 1024);
-                nl = *reinterpret_cast<const bf16x8*>(st + GD_OPB + ro + (i + 1) * 1024);
+                nl = *reinterpret_cast<const bf16x8*>(st + AOP + ro + (i + 1) * 1024);
             }
-            if constexpr (decltype(MORE)::value) {   // the 12 blocks over the 8 row tiles: two, one, two, ...
-                dma(kt + 2, 3 * (i / 2) + 2 * (i & 1));
-                if (!(i & 1)) dma(kt + 2, 3 * (i / 2) + 1);
+            if constexpr (more) {   // the NB blocks spread over the TI row tiles
+#pragma unroll
+                for (int b = i * NB / TI; b < (i + 1) * NB / TI; ++b) dma(kt + 2, b);
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[j], acc[i][j], 0, 0, 0);
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TJ; ++j) {
+                if constexpr (QUANT) {
+                    floatx4 t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[j], floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[j], t, 0, 0, 0);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(sc[j], t[r], acc[i][j][r]);
+                } else {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[j], acc[i][j], 0, 0, 0);
+                    if constexpr (TYPE == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[j], acc[i][j], 0, 0, 0);
+                }
             }
             ah = nh;
             al = nl;
         }
     };
     uint32_t kt = 0;
-    for (; kt + 2 < nk; ++kt) step(kt, std::integral_constant<bool, true>{});
-    for (; kt < nk; ++kt) step(kt, std::integral_constant<bool, false>{});
+    for (; kt + 2 < kSteps; ++kt) step(kt, std::bool_constant<true>{});
+    for (; kt < kSteps; ++kt) step(kt, std::bool_constant<false>{});
     // the accumulator layout: lane holds rows 4 (lane / 16) + r of column lane % 16
+    float* const out = a.part ? a.part + size_t(blockIdx.y) * M * a.columns + n0 : S.out + wn0;
+    const uint32_t ldo = a.part ? a.columns : S.ldo;
+    const bool add = a.accumulate && !a.part;   // a K slice: its own partial (no bias, no accumulate)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const uint32_t n = n0 + 128 * wn + 16 * j + fr;
-        if (n >= N) continue;
-        const float b = p.bias ? p.bias[n] : 0.0f;
+    for (int j = 0; j < TJ; ++j) {
+        const uint32_t c = BN / WN * wn + 16 * j + fr;
+        if (wn0 + c >= S.n) continue;
+        const float b = S.bias && !a.part ? S.bias[wn0 + c] : 0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < TI; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const uint32_t m = m0 + 128 * wm + 16 * i + 4 * (lane >> 4) + r;
+                const uint32_t m = m0 + BM / 2 * wm + 16 * i + 4 * g + r;
                 if (m >= M) continue;
-                float* o = p.out + size_t(m) * p.ldo + n;
-                *o = (p.accumulate ? *o : 0.0f) + acc[i][j][r] + b;
+                float* o = out + size_t(m) * ldo + c;
+                *o = (add ? *o : 0.0f) + acc[i][j][r] + b;
             }
+    }
+}
+
+/* the K slices' partial tiles added in slice order, then the bias and the
+   accumulate */
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, uint32_t slices) {
+    const uint64_t quads = uint64_t(a.m) * a.columns / 4, slice = uint64_t(a.m) * a.columns;
+    for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < quads; i += uint64_t(gridDim.x) * 256) {
+        const uint32_t m = uint32_t(4 * i / a.columns), n = uint32_t(4 * i % a.columns);
+        const GemmSeg& S = a.seg[segment_of(a, n)];
+        const uint32_t c = n - S.start;
+        if (c >= S.n) continue;
+        floatx4 v = {0.0f, 0.0f, 0.0f, 0.0f};   // columns past n were not written: not used below
+        for (uint32_t sl = 0; sl < slices; ++sl) {
+            const floatx4 x = *reinterpret_cast<const floatx4*>(a.part + sl * slice + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += x[e];
+        }
+        float* o = S.out + size_t(m) * S.ldo + c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (c + e < S.n) o[e] = (a.accumulate ? o[e] : 0.0f) + v[e] + (S.bias ? S.bias[c + e] : 0.0f);
     }
 }
 
@@ -663,29 +726,110 @@ __global__ __launch_bounds__(256) void gemv_scalar_kernel(GemvParams p) {
     }
 }
 
-/* bf16 weights with at least 256 tiles of 256 x 256 (a and w under 4 GB,
-   k a multiple of 32) take split_a_kernel and gemm_dma_kernel */
+constexpr uint32_t CUS = 256;
+
+/* shapes gemm_dma_kernel takes: K in whole steps (of four for Q8 and Q4, whose
+   scales come in four at a time), 16-byte aligned rows, 32-bit byte offsets */
 bool dma_eligible(const GemvParams& p) {
-    // at least half a 256-row tile of a: fewer rows (a decode step's GEMV
-    // against a wide weight such as an LM head) would waste most of every tile
-    if (p.type != 1 || p.m < GD_BM / 2 || p.k % GD_BK || (reinterpret_cast<uintptr_t>(p.w) % 16) ||
-        (reinterpret_cast<uintptr_t>(p.a) % 16))
+    auto aligned = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) % 16) == 0; };
+    if (p.m < GEMM_MIN_M || p.k % (p.type >= 2 ? 4 * GD_BK : GD_BK) || !aligned(p.w) || !aligned(p.a) ||
+        (p.type >= 2 && !aligned(p.scales)))
         return false;
-    const uint64_t wide = uint64_t((p.m + GD_BM - 1) / GD_BM) * ((p.n + GD_BN - 1) / GD_BN);
-    return wide >= 256 && wide <= 0x7FFFFFFFull && uint64_t(p.m) * p.k * 2 < (1ull << 32) &&
-           uint64_t(p.n) * p.k * 2 < (1ull << 32);
+    const uint64_t rowBytes = uint64_t(p.k) / GD_BK * (p.type == 0 ? 128 : (p.type == 1 ? 64 : (p.type == 2 ? 32 : 16)));
+    return uint64_t(p.m) * p.k * 2 < (1ull << 32) && uint64_t(p.n) * rowBytes < (1ull << 32) && p.m <= 0x7FFFFFFFu / 2;
 }
 
-/* a split into its bf16 high parts and residuals (scratch slot SLOT_GEMM_A),
-   unless `split` says the slot already holds them, then the DMA GEMM; w2 /
-   nSplit as gemm_dma_kernel */
-bool launch_dma(Context& ctx, const GemvParams& p, const void* w2, uint32_t nSplit, bool split, hipStream_t stream) {
-    const uint64_t wide = uint64_t((p.m + GD_BM - 1) / GD_BM) * ((p.n + GD_BN - 1) / GD_BN);
+struct GemmPlan {
+    int bm, bn;
+    uint32_t tiles, slices, sliceSteps, columns;
+};
+
+/* The tile and the number of K slices by estimated time, from what each tile
+   costs per 32-wide K step (microseconds, measured at k = 4096, m 16 to 8192,
+   n 2048 to 12288): `alone` on its CU with the others idle, `shared` for each
+   of several on one CU, or with every CU busy (the clock falls, L2 fills up).
+   Small tiles and K slices win while the tiles of one shape do not fill 256
+   CUs (m = 500, k = n = 4096, bf16: 256 x 256 tiles 169 us, 128 x 128 71, two
+   K slices 57), large ones by their reuse when they do (m = 8192: 450, 128 x
+   256 502, 128 x 128 557). Slices cost their partial tiles' round trip. */
+struct TileCost {
+    int type, bm, bn, resident;   // workgroups of this tile a CU's LDS holds
+    float alone, shared;
+};
+constexpr TileCost TILE_COSTS[] = {
+    {0, 128, 256, 1, 1.22f, 1.43f}, {0, 128, 128, 1, 0.68f, 0.80f}, {0, 64, 128, 2, 0.62f, 0.55f},
+    {1, 256, 256, 1, 1.26f, 1.66f}, {1, 128, 256, 1, 0.77f, 0.93f}, {1, 128, 128, 2, 0.49f, 0.51f}, {1, 64, 128, 3, 0.30f, 0.31f},
+    {2, 128, 256, 1, 0.98f, 1.10f}, {2, 128, 128, 2, 0.72f, 0.58f}, {2, 64, 128, 3, 0.53f, 0.39f},
+    {3, 128, 128, 2, 0.82f, 0.64f}, {3, 64, 128, 4, 0.62f, 0.46f},
+};
+
+GemmPlan plan_gemm(const GemvParams* ps, int count) {
+    const GemvParams& p = ps[0];
+    GemmPlan best{};
+    float bestCost = 0.0f;
+    const uint32_t steps = p.k / GD_BK, group = p.type >= 2 ? 4 : 1;
+    for (const TileCost& t : TILE_COSTS) {
+        if (t.type != p.type) continue;
+        uint64_t columns = 0;
+        for (int i = 0; i < count; ++i) columns += (ps[i].n + t.bn - 1) / t.bn;
+        const uint64_t tiles = uint64_t((p.m + t.bm - 1) / t.bm) * columns;
+        columns *= t.bn;
+        if (tiles > 0x7FFFFFFFull || columns > 0x7FFFFFFFull) continue;
+        for (uint32_t want = 1; want <= 16; want = want < 4 ? want + 1 : want + 2) {
+            const uint32_t per = ((steps + want - 1) / want + group - 1) / group * group;   // whole scale groups
+            if ((steps + per - 1) / per != want || (want > 1 && per < 8)) continue;
+            // rounds of `resident` tiles a CU; a last round's tiles land where
+            // CUs fall free, several on one while others have none
+            const uint64_t items = tiles * want, round = uint64_t(CUS) * t.resident;
+            const uint64_t rounds = (items + round - 1) / round, most = (items + CUS - 1) / CUS;
+            const float full = items < CUS ? float(items) / CUS : 1.0f;
+            const float lastFill = float(items - (rounds - 1) * round) / float(round);
+            float step = t.alone + (t.shared > t.alone ? (t.shared - t.alone) * full : 0.0f);
+            if (rounds == 1 && most > 1) step = fmaxf(t.alone, float(most) * t.shared);
+            if (rounds > 1) step = (float(rounds - 1) + (t.resident == 1 ? 1.0f : 0.6f + 0.4f * lastFill)) * float(t.resident) * t.shared;
+            float cost = step * per + 1.5f * float(rounds);
+            if (want > 1) cost += 4.0f + float(want) * float(p.m) * float(columns) * 8.0f / 6e6f;
+            if (best.bm == 0 || cost < bestCost) {
+                best = GemmPlan{t.bm, t.bn, uint32_t(tiles), want, per, uint32_t(columns)};
+                bestCost = cost;
+            }
+        }
+    }
+    return best;
+}
+
+/* the products of one a with `count` weights (same a, m, k, type and
+   accumulate): a split into its bf16 high parts and residuals (scratch slot
+   SLOT_GEMM_A), unless `split` says the slot already holds them, then the DMA
+   GEMM. A plan with K slices writes partial tiles that gemm_reduce_kernel adds
+   in order. */
+bool launch_dma(Context& ctx, const GemvParams* ps, int count, bool split, hipStream_t stream) {
+    const GemvParams& p = ps[0];
     const uint64_t aBytes = uint64_t(p.m) * p.k * 2;   // one bf16 image of a
     uint8_t* img = static_cast<uint8_t*>(ctx.grow(SLOT_GEMM_A, 2 * aBytes));
     if (!img) return false;
     bf16x8* hi = reinterpret_cast<bf16x8*>(img);
     bf16x8* lo = reinterpret_cast<bf16x8*>(img + aBytes);
+    const GemmPlan plan = plan_gemm(ps, count);
+    if (plan.bm == 0) return ctx.fail("matmul: too many tiles");
+    GemmArgs a{};
+    a.ahi = reinterpret_cast<const __bf16*>(hi);
+    a.alo = reinterpret_cast<const __bf16*>(lo);
+    uint32_t start = 0;
+    for (int i = 0; i < count; ++i) {
+        a.seg[i] = GemmSeg{ps[i].w, ps[i].scales, ps[i].bias, ps[i].out, ps[i].n, ps[i].ldo, start};
+        start += (ps[i].n + plan.bn - 1) / plan.bn * plan.bn;
+    }
+    a.nseg = uint32_t(count);
+    a.m = p.m;
+    a.k = p.k;
+    a.accumulate = p.accumulate ? 1u : 0u;
+    a.columns = plan.columns;
+    a.sliceSteps = plan.sliceSteps;
+    if (plan.slices > 1) {
+        a.part = static_cast<float*>(ctx.grow(SLOT_GEMM_SPLIT, size_t(plan.slices) * p.m * plan.columns * sizeof(float)));
+        if (!a.part) return false;
+    }
     if (!split) {
         const uint64_t pieces = aBytes / 16;
         const unsigned sg = unsigned((pieces + 255) / 256 < 8192 ? (pieces + 255) / 256 : 8192);
@@ -694,9 +838,31 @@ bool launch_dma(Context& ctx, const GemvParams& p, const void* w2, uint32_t nSpl
             }))
             return false;
     }
-    return ctx.launch("gemm_dma_kernel", stream, [&] {
-        hipLaunchKernelGGL(gemm_dma_kernel, dim3(unsigned(wide)), dim3(256), 0, stream, p,
-                           reinterpret_cast<const __bf16*>(hi), reinterpret_cast<const __bf16*>(lo), w2, nSplit);
+    const dim3 grid(plan.tiles, plan.slices);
+    if (!ctx.launch("gemm_dma_kernel", stream, [&] {
+#define AIGPU_GD(T, BM, BN, WN)                             \
+    if (p.type == T && plan.bm == BM && plan.bn == BN)      \
+        hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WN>), grid, dim3(128 * WN), 0, stream, a)
+            AIGPU_GD(0, 128, 256, 4);
+            AIGPU_GD(0, 128, 128, 4);
+            AIGPU_GD(0, 64, 128, 2);
+            AIGPU_GD(1, 256, 256, 4);
+            AIGPU_GD(1, 128, 256, 4);
+            AIGPU_GD(1, 128, 128, 2);
+            AIGPU_GD(1, 64, 128, 2);
+            AIGPU_GD(2, 128, 256, 4);
+            AIGPU_GD(2, 128, 128, 2);
+            AIGPU_GD(2, 64, 128, 2);
+            AIGPU_GD(3, 128, 128, 2);
+            AIGPU_GD(3, 64, 128, 2);
+#undef AIGPU_GD
+        }))
+        return false;
+    if (plan.slices == 1) return true;
+    const uint64_t quads = uint64_t(p.m) * plan.columns / 4;
+    const unsigned rg = unsigned((quads + 255) / 256 < 65536 ? (quads + 255) / 256 : 65536);
+    return ctx.launch("gemm_reduce_kernel", stream, [&] {
+        hipLaunchKernelGGL(gemm_reduce_kernel, dim3(rg), dim3(256), 0, stream, a, plan.slices);
     });
 }
 
@@ -713,9 +879,7 @@ bool launch_type(Context& ctx, const GemvParams& p, hipStream_t stream) {
         }
         return ctx.fail("matmul: quantised weights need k a multiple of 32 and 16-byte aligned rows");
     }
-    if constexpr (TYPE == 1) {
-        if (dma_eligible(p)) return launch_dma(ctx, p, nullptr, 0, false, stream);
-    }
+    if (dma_eligible(p)) return launch_dma(ctx, &p, 1, false, stream);
     if (p.m >= GEMM_MIN_M) {
         const uint32_t tiles = ((p.n + GM_BN - 1) / GM_BN) * ((p.m + GM_BM - 1) / GM_BM);
         // fewer tiles than CUs and a long K: split K into slices of at least
@@ -733,7 +897,7 @@ bool launch_type(Context& ctx, const GemvParams& p, hipStream_t stream) {
         if (grid.y > 65535u) return ctx.fail("matmul: too many rows of a");
         if (slices == 1)
             return ctx.launch("gemm_kernel", stream, [&] {
-                hipLaunchKernelGGL((gemm_kernel<TYPE, false>), grid, dim3(256), 0, stream, p, KvEpilogue{}, kSlice);
+                hipLaunchKernelGGL((gemm_kernel<TYPE>), grid, dim3(256), 0, stream, p, kSlice);
             });
         float* part = static_cast<float*>(ctx.grow(SLOT_GEMM_SPLIT, size_t(slices) * p.m * p.n * sizeof(float)));
         if (!part) return false;
@@ -743,7 +907,7 @@ bool launch_type(Context& ctx, const GemvParams& p, hipStream_t stream) {
         q.bias = nullptr;
         q.accumulate = 0;
         if (!ctx.launch("gemm_kernel", stream, [&] {
-                hipLaunchKernelGGL((gemm_kernel<TYPE, false>), grid, dim3(256), 0, stream, q, KvEpilogue{}, kSlice);
+                hipLaunchKernelGGL((gemm_kernel<TYPE>), grid, dim3(256), 0, stream, q, kSlice);
             }))
             return false;
         const uint64_t outs = uint64_t(p.m) * p.n;
@@ -766,6 +930,21 @@ bool launch_type(Context& ctx, const GemvParams& p, hipStream_t stream) {
 }
 
 } // namespace
+
+bool launch_gemvs(const GemvParams* ps, int count, bool split, hipStream_t stream) {
+    Context& ctx = Context::instance();
+    bool together = count <= GD_SEGS;
+    for (int i = 0; i < count; ++i) {
+        const GemvParams &p = ps[i], &f = ps[0];
+        together = together && p.a == f.a && p.m == f.m && p.k == f.k && p.type == f.type &&
+                   (p.accumulate != 0) == (f.accumulate != 0) && p.n > 0 && p.ldo >= p.n && p.w && p.out &&
+                   (p.type < 2 || p.scales) && p.type >= 0 && p.type <= 3 && p.a && dma_eligible(p);
+    }
+    if (together && count > 0) return launch_dma(ctx, ps, count, split, stream);
+    for (int i = 0; i < count; ++i)
+        if (!launch_gemv(ps[i], stream)) return false;
+    return true;
+}
 
 bool launch_gemv(const GemvParams& p, hipStream_t stream) {
     Context& ctx = Context::instance();
@@ -797,32 +976,29 @@ bool launch_gemv_presplit(const GemvParams& p, hipStream_t stream) {
     Context& ctx = Context::instance();
     if (p.m == 0 || p.n == 0) return true;
     if (!p.w || !p.out || p.ldo < p.n || !dma_eligible(p)) return ctx.fail("matmul: no presplit GEMM for this shape");
-    return launch_dma(ctx, p, nullptr, 0, true, stream);
+    return launch_dma(ctx, &p, 1, true, stream);
 }
 
 bool launch_gemm_kv_pair(const GemvParams& pk, const GemvParams& pv, const KvEpilogue& ek, const KvEpilogue& ev,
                          bool aSplit, bool fold, float* rope, bool* folded, hipStream_t stream) {
     Context& ctx = Context::instance();
     *folded = false;
-    // one DMA GEMM over both weights when each is a multiple of 256 columns
-    // (no tile straddles them) and the pair has the tiles for it
-    GemvParams both = pk;
-    both.n = pk.n + pv.n;
-    both.ldo = both.n;
-    both.bias = nullptr;
-    both.accumulate = 0;
-    const bool pair = pk.type == 1 && pv.type == 1 && pk.k == pv.k && pk.m == pv.m && pk.a == pv.a && pk.n == pv.n &&
-                      pk.n % GD_BN == 0 && (ek.dim == 64 || ek.dim == 128) && ek.dim == ev.dim &&
-                      (reinterpret_cast<uintptr_t>(pv.w) % 16) == 0 && dma_eligible(both);
-    if (!pair) return launch_gemm_kv(pk, ek, stream) && launch_gemm_kv(pv, ev, stream);
     if (pk.m == 0) return true;
     if (!kv_checks(ctx, pk, ek) || !kv_checks(ctx, pv, ev)) return false;
-    float* kv = static_cast<float*>(ctx.grow(SLOT_MIXER_KV, size_t(pk.m) * both.n * sizeof(float)));
+    if (pk.n != pv.n || pk.m != pv.m || pk.a != pv.a || ek.dim != ev.dim)
+        return ctx.fail("projection epilogue: k and v differ in shape");
+    // k and v side by side, [m][k's columns, v's]
+    float* kv = static_cast<float*>(ctx.grow(SLOT_MIXER_KV, size_t(pk.m) * 2 * pk.n * sizeof(float)));
     if (!kv) return false;
-    both.out = kv;
-    if (!launch_dma(ctx, both, pv.w, pk.n, aSplit, stream)) return false;
+    GemvParams both[2] = {pk, pv};
+    for (int i = 0; i < 2; ++i) {
+        both[i].out = kv + i * pk.n;
+        both[i].ldo = 2 * pk.n;
+        both[i].bias = nullptr;
+        both[i].accumulate = 0;
+    }
+    if (!launch_gemvs(both, 2, aSplit, stream)) return false;
     const uint32_t heads = pk.n / ek.dim;
-    if (pk.m > 0x7FFFFFFFu) return ctx.fail("projection epilogue: too many rows");
     if (fold && rope && !ek.freqs) return ctx.fail("projection epilogue: a cos/sin table needs RoPE");
     // the pad rows start past the last head's T rows (16-byte aligned: dim is 64 or 128)
     const size_t padAt = size_t(heads) * ek.T * ek.dim * 2;
@@ -852,22 +1028,6 @@ static bool kv_checks(Context& ctx, const GemvParams& p, const KvEpilogue& e) {
         (reinterpret_cast<uintptr_t>(e.cache) % 16) || (reinterpret_cast<uintptr_t>(e.work) % 16))
         return ctx.fail("projection epilogue: rows of a, w and the caches must be 16-byte aligned");
     return true;
-}
-
-bool launch_gemm_kv(const GemvParams& p, const KvEpilogue& e, hipStream_t stream) {
-    Context& ctx = Context::instance();
-    if (p.m == 0) return true;
-    if (!kv_checks(ctx, p, e)) return false;
-    const dim3 grid(unsigned((p.n + GM_BN - 1) / GM_BN), unsigned((p.m + GM_BM - 1) / GM_BM));
-    if (grid.y > 65535u) return ctx.fail("matmul: too many rows of a");
-    return ctx.launch("gemm_kv_kernel", stream, [&] {
-        switch (p.type) {
-            case 0: hipLaunchKernelGGL((gemm_kernel<0, true>), grid, dim3(256), 0, stream, p, e, p.k + GM_BK); break;
-            case 1: hipLaunchKernelGGL((gemm_kernel<1, true>), grid, dim3(256), 0, stream, p, e, p.k + GM_BK); break;
-            case 2: hipLaunchKernelGGL((gemm_kernel<2, true>), grid, dim3(256), 0, stream, p, e, p.k + GM_BK); break;
-            default: hipLaunchKernelGGL((gemm_kernel<3, true>), grid, dim3(256), 0, stream, p, e, p.k + GM_BK); break;
-        }
-    });
 }
 
 } // namespace aigpu

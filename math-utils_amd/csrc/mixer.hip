@@ -3,10 +3,9 @@
 // QK-RMSNorm -> RoPE -> KV append, causal attention over the cache, the
 // output gate, and the o projection.
 //
-// The k and v projections carry the per-token work as their GEMM's epilogue
-// (launch_gemm_kv): the normed, rotated rows go straight from the MFMA
-// accumulators to the bf16 cache and to the flash kernel's fp16 copy, with
-// no fp32 k / v round trip through HBM and no separate prep pass over them.
+// The k and v projections go as one GEMM into scratch, and one pass over its
+// rows norms, rotates and appends them to the bf16 cache and to the flash
+// kernel's fp16 copy.
 // The q projection is stored raw: the flash kernel normalises and rotates
 // its own q rows on load (or prep does, when the shape rules that out).
 #include "context.hpp"

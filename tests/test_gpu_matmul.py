@@ -1,6 +1,6 @@
-"""GPU parity of the projections (gemv_kernel for up to 15 rows of a,
-gemm_kernel on MFMA from 16, split_a_kernel and gemm_dma_kernel for bf16
-weights with enough 256 x 256 tiles, behind aigpu_matmul_nt* and
+"""GPU parity of the projections (gemv_kernel for up to 15 rows of a, from 16
+split_a_kernel and gemm_dma_kernel on MFMA, gemm_kernel for the k that one
+does not take, behind aigpu_matmul_nt* and
 aigpu_matmul_device)
 against the oracle's restatement of apply
 (LocalModel.hpp:1052-1078) over the reference's weight encodings.
@@ -205,3 +205,25 @@ def test_one_row_against_a_wide_weight_takes_the_gemv(gpu):
     assert gpu.profile_read("gemm_dma_kernel")[1] == 0
     err = np.abs(host(out) - O.matmul_nt(a, w, "bf16"))
     assert np.all(err <= bound(a, dense)), f"max err {err.max()}"
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8", "q4"])
+@pytest.mark.parametrize("m,n,k", [(17, 130, 128), (65, 257, 640), (300, 1100, 384), (1030, 3000, 128), (2001, 4000, 256)])
+def test_gemm_dma_tiles(gpu, kind, m, n, k):
+    """gemm_dma_kernel at sizes from a part of its smallest tile to enough of its
+    largest, every tile row and column ragged: m, n one past or short of a
+    multiple, K of one group of four steps up, with and without K slices"""
+    import torch
+    a = O.fill_normal((m, k), 71 + m, "a")
+    w, scales, dense = weights(n, k, kind, 72 + n)
+    base = O.fill_normal((m, n + 3), 73, "base")
+    out = dev_f32(base)
+    say("gemm dma", dict(kind=kind, m=m, k=k, n=n))
+    gpu.matmul(dev_f32(a), to_device(w), out[:, :n], kind, scales=None if scales is None else dev_f32(scales),
+               accumulate=True)
+    got = host(out)
+    want = base[:, :n] + O.matmul_nt(a, w, kind, scales=scales)
+    err = np.abs(got[:, :n] - want)
+    # the bar of this file, plus the residual add's own rounding
+    assert np.all(err <= bound(a, dense) + 1e-6 * (1 + np.abs(base[:, :n]))), f"{kind}: max err {err.max()}"
+    np.testing.assert_array_equal(got[:, n:], base[:, n:])
