@@ -1,16 +1,17 @@
 // indexer.hip - the sparse-attention indexer (selectKeys, LocalModel.hpp:
 // 2971-3068) in GLM-5.3's pooled form, on the device. Per call of `count`
 // tokens at startPos:
-//   projections        k = idxK h, gates = idxGate h (into the gate cache),
-//                      and, when some token is sparse, q = idxQB qResid and
-//                      w = idxWeights h (launch_gemv)
+//   projections        k = idxK h, gates = idxGate h (into the gate cache)
+//                      and, when some token is sparse, w = idxWeights h in
+//                      one launch (launch_gemvs), q = idxQB qResid
 //   index_norm_kernel  layerNormRow (:1355-1367, eps 1e-6) of each k into
 //                      the key cache (:2988-2990)
 //   index_pool_kernel  every pool a token of the call completes: per channel
 //                      the softmax over its members of gate + ape, applied
 //                      to their keys (:2994-3009)
-//   index_score_kernel per sparse token and pool wholly at or before it:
-//                      sum over heads of w headScale relu(q . pool dimScale)
+//   index_score_mfma_kernel, index_score_kernel (index heads over 128)
+//                      per sparse token and pool wholly at or before it: sum
+//                      over heads of w headScale relu(q . pool dimScale)
 //                      (:3038-3047)
 //   index_select_kernel per token: the topK / P best pools by radix select
 //                      on the scores' order-preserving bits, expanded to
@@ -147,6 +148,212 @@ __global__ __launch_bounds__(256) void index_score_kernel(IndexArgs a, const flo
             scores[size_t(t) * a.maxPools + p] = s;
         }
         __syncthreads();   // part is rewritten by the next block
+    }
+}
+
+/*
+    index_score_mfma_kernel: the same scores on the matrix cores, for index
+    heads of up to 128 (every model's). A wave holds four row tiles of 16 heads
+    (HT tiles per token, so 4 / HT tokens) of q as MFMA A operands in registers
+    for the whole launch; the workgroup's WT x WP waves take WT such token
+    groups and share blocks of 64 pools in LDS (each wave 64 / WP of a block's
+    pools). q and the pools are fp32: each row is scaled by a power of two to a
+    largest element in [2^10, 2^11) and split into two fp16 terms (22 bits),
+    and q.pool is three products, hi.hi + hi.lo + lo.hi, added in fp32 32
+    channels at a time. The terms left out are below 2^-22 of their product and
+    the sum is rounded four times instead of 128, so the dots carry less error
+    than the fp32 chain's (scores against float64, 1 to 500 tokens of 16 x 64
+    to 64 x 128 heads: 0.72 to 0.76 of it). relu commutes with the (positive) scales, so a lane
+    applies w headScale / scale_q once per head and dimScale / scale_pool once
+    per pool. A row that is not finite has no such split: its scores are formed
+    as index_score_kernel forms them.
+    Bound by the MFMAs (48 per 16 pools and wave, 8 KB of LDS reads):
+    1024 tokens x 2,006 pools, 64 x 128: 1045 us with index_score_kernel (fp32
+    FMA against LDS broadcasts), 120 us here; a decode step at 8,192 pools, the
+    whole call: 91 and 86 us.
+*/
+constexpr int IXM_DIM = 128, IXM_BLOCK = 64, IXM_KS = IXM_DIM / 32;
+
+/* the exponent se with max 2^se in [2^10, 2^11) (at most 127; 0 for a zero row) */
+__device__ __forceinline__ int split_exponent(float mx) {
+    const int e = int(__float_as_uint(mx) >> 23);
+    return mx == 0.0f ? 0 : (137 - e > 127 ? 127 : 137 - e);
+}
+
+/* eight scaled values as two fp16 terms */
+__device__ __forceinline__ void split_half(const float (&x)[8], float scale, half8& hi, half8& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float y = x[e] * scale;
+        hi[e] = _Float16(y);
+        lo[e] = _Float16(y - float(hi[e]));
+    }
+}
+
+template <int HT, int WT, int WP>
+__global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(IndexArgs a, const float* q, const float* w,
+                                                                          const float* pools, float* scores) {
+    constexpr int THREADS = 64 * WT * WP, TPW = 4 / HT;          // tokens per wave
+    constexpr int PIECES = IXM_BLOCK * IXM_DIM / 8 / THREADS;    // 8-channel pieces per thread and block
+    constexpr int IMG = IXM_BLOCK * IXM_DIM;                     // halves of one image of a block
+    __shared__ __align__(16) _Float16 img[2][2 * IMG];           // [buffer][hi, lo]
+    __shared__ float inv[2][IXM_BLOCK];                          // dimScale 2^-se of each pool, NaN: not finite
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wt = wv / WP, wp = wv % WP;
+    const uint32_t nI = a.nI, Di = a.Di;
+    const uint32_t t0 = (blockIdx.x * WT + wt) * TPW;            // the wave's first token
+    const uint32_t gLast = (blockIdx.x + 1) * WT * TPW < a.count ? (blockIdx.x + 1) * WT * TPW : a.count;
+    // the group's last token sees the most pools; a token that needs no scores
+    // sees fewer than one that does
+    const uint32_t most = (a.startPos + gLast) / a.P;
+    if (sees_everything(a, most) || blockIdx.y * IXM_BLOCK >= most) return;   // uniform, before any barrier
+
+    // q rows as A operands: lane (c16, g) holds row c16, channels 32 s + 8 g .. + 7
+    half8 ah[4][IXM_KS], al[4][IXM_KS];
+    float coef[4][4];   // w headScale 2^-se of the accumulator's rows 4 g + r
+    bool badQ = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t t = t0 + i / HT, h = 16 * (i % HT) + c16;
+        const bool live = t < a.count && h < nI;
+        float x[IXM_KS][8], mx = 0.0f;
+        bool finite = true;
+#pragma unroll
+        for (int s = 0; s < IXM_KS; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const uint32_t d = 32 * s + 8 * g + e;
+                const floatx4 v = live && d < Di ? *reinterpret_cast<const floatx4*>(q + (size_t(t) * nI + h) * Di + d)
+                                                 : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    x[s][e + c] = v[c];
+                    mx = fmaxf(mx, fabsf(v[c]));
+                    finite = finite && fabsf(v[c]) < INFINITY;
+                }
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        const int se = split_exponent(mx);
+        const float scale = ldexpf(1.0f, se);
+#pragma unroll
+        for (int s = 0; s < IXM_KS; ++s) split_half(x[s], scale, ah[i][s], al[i][s]);
+        badQ = badQ || !finite;
+        const float wh = live ? w[size_t(t) * nI + h] * a.headScale * ldexpf(1.0f, -se) : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) coef[i][r] = __shfl(wh, 4 * g + r, WAVE);   // lane 4 g + r holds that row
+    }
+    badQ = __any(badQ);
+
+    // a block's pools: thread piece j is row (tid + THREADS j) / 16, channels 8 (tid % 16) ..
+    float px[PIECES][8];
+    auto load = [&](uint32_t p0) {
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j) {
+            const uint32_t idx = tid + THREADS * j, p = p0 + idx / 16, d = 8 * (idx % 16);
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const floatx4 v = p < most && d + e < Di ? *reinterpret_cast<const floatx4*>(pools + size_t(p) * Di + d + e)
+                                                         : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) px[j][e + c] = v[c];
+            }
+        }
+    };
+    // rows of 16 chunks of 8 halves; chunk c of row r at c ^ (r % 16), so the 16
+    // rows an operand read takes lie on distinct banks
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j) {
+            const uint32_t idx = tid + THREADS * j, row = idx / 16, c = idx % 16;
+            float mx = 0.0f;
+            uint32_t bad = 0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                mx = fmaxf(mx, fabsf(px[j][e]));
+                bad |= fabsf(px[j][e]) < INFINITY ? 0u : 1u;
+            }
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) {
+                mx = fmaxf(mx, __shfl_xor(mx, o, WAVE));
+                bad |= __shfl_xor(bad, o, WAVE);
+            }
+            const int se = split_exponent(mx);
+            half8 hi, lo;
+            split_half(px[j], ldexpf(1.0f, se), hi, lo);
+            const uint32_t at = row * IXM_DIM + 8 * (c ^ (row & 15));
+            *reinterpret_cast<half8*>(&img[buf][at]) = hi;
+            *reinterpret_cast<half8*>(&img[buf][IMG + at]) = lo;
+            if (c == 0) inv[buf][row] = bad ? __builtin_nanf("") : a.dimScale * ldexpf(1.0f, -se);
+        }
+    };
+
+    uint32_t p0 = blockIdx.y * IXM_BLOCK;
+    const uint32_t stride = gridDim.y * IXM_BLOCK;
+    load(p0);
+    store(0);
+    __syncthreads();
+    for (int buf = 0; p0 < most; p0 += stride, buf ^= 1) {   // uniform
+        if (p0 + stride < most) load(p0 + stride);
+#pragma unroll 1
+        for (int ct = wp; ct < IXM_BLOCK / 16; ct += WP) {
+            const int row = 16 * ct + c16;
+            half8 bh[IXM_KS], bl[IXM_KS];
+#pragma unroll
+            for (int s = 0; s < IXM_KS; ++s) {
+                const uint32_t at = row * IXM_DIM + 8 * ((4 * s + g) ^ c16);
+                bh[s] = *reinterpret_cast<const half8*>(&img[buf][at]);
+                bl[s] = *reinterpret_cast<const half8*>(&img[buf][IMG + at]);
+            }
+            const float ip = inv[buf][row];
+            floatx4 acc[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < IXM_KS; ++s) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i][s], bl[s], acc[i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i][s], bh[s], acc[i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i][s], bh[s], acc[i], 0, 0, 0);
+            }
+            // relu, the head weights, and the sum over a token's heads: the
+            // lane's four rows of each tile, then the four lane groups
+            float sum[TPW];
+#pragma unroll
+            for (int tk = 0; tk < TPW; ++tk) {
+                float v = 0.0f;
+#pragma unroll
+                for (int i = tk * HT; i < (tk + 1) * HT; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v = fmaf(coef[i][r], fmaxf(acc[i][r], 0.0f), v);
+                v += __shfl_xor(v, 16, WAVE);
+                v += __shfl_xor(v, 32, WAVE);
+                sum[tk] = v * ip;
+            }
+            const uint32_t p = p0 + row;
+            const bool slow = badQ || !(ip == ip);
+#pragma unroll
+            for (int tk = 0; tk < TPW; ++tk) {
+                const uint32_t t = t0 + tk, complete = t < a.count ? (a.startPos + t + 1) / a.P : 0u;
+                if (g != 0 || p >= complete || sees_everything(a, complete)) continue;
+                float out = sum[tk];
+                if (slow) {   // a value that is not finite: the fp32 chain of index_score_kernel
+                    out = 0.0f;
+                    for (uint32_t h = 0; h < nI; ++h) {
+                        float d = 0.0f;
+                        for (uint32_t k = 0; k < Di; ++k)
+                            d = fmaf(q[(size_t(t) * nI + h) * Di + k], pools[size_t(p) * Di + k], d);
+                        const float logit = d * a.dimScale;
+                        out += w[size_t(t) * nI + h] * a.headScale * (logit > 0.0f ? logit : 0.0f);
+                    }
+                }
+                scores[size_t(t) * a.maxPools + p] = out;
+            }
+        }
+        if (p0 + stride < most) store(buf ^ 1);   // the other buffer's reads ended before the last barrier
+        __syncthreads();
     }
 }
 
@@ -344,8 +551,11 @@ bool launch_select_keys(const IndexerParams& p, hipStream_t stream) {
     float* scores = p.scores ? p.scores : reinterpret_cast<float*>(work + align(kBytes) + align(qBytes) + align(wBytes));
 
     const uint32_t m = uint32_t(p.count);
-    if (!launch_gemv(projection(p.wk, p.h, k, m, uint32_t(Di)), stream)) return false;
-    if (!launch_gemv(projection(p.wgate, p.h, p.gates + p.startPos * Di, m, uint32_t(Di)), stream)) return false;
+    // the projections of h together: k, the gates and, when some token is sparse, w
+    const GemvParams ofH[3] = {projection(p.wk, p.h, k, m, uint32_t(Di)),
+                               projection(p.wgate, p.h, p.gates + p.startPos * Di, m, uint32_t(Di)),
+                               projection(p.ww, p.h, w, m, uint32_t(nI))};
+    if (!launch_gemvs(ofH, anySparse ? 3 : 2, false, stream)) return false;
 
     IndexArgs a{};
     a.count = m;
@@ -372,9 +582,28 @@ bool launch_select_keys(const IndexerParams& p, hipStream_t stream) {
         return false;
     if (anySparse) {
         if (!launch_gemv(projection(p.wq, p.qResid, q, m, uint32_t(nI * Di)), stream)) return false;
-        if (!launch_gemv(projection(p.ww, p.h, w, m, uint32_t(nI)), stream)) return false;
         if (maxPools > 0 &&
             !ctx.launch("index_score_kernel", stream, [&] {
+                if (Di <= uint64_t(IXM_DIM)) {
+                    // eight waves of 4 / HT tokens each share a block of pools;
+                    // few tokens: four waves share their tokens and split the block
+                    const uint64_t blocks = (maxPools + IXM_BLOCK - 1) / IXM_BLOCK;
+                    const int ht = nI <= 16 ? 1 : (nI <= 32 ? 2 : 4);
+                    const bool few = m <= 16u / ht;
+                    const uint32_t perGroup = (few ? 4u : 32u) / ht, groups = (m + perGroup - 1) / perGroup;
+                    const uint64_t want = few ? (1024 + groups - 1) / groups : (512 + groups - 1) / groups;
+                    const dim3 grid(groups, unsigned(blocks < want ? blocks : want));
+#define AIGPU_IX(HT)                                                                                                \
+    if (ht == HT) {                                                                                                 \
+        if (few)                                                                                                    \
+            hipLaunchKernelGGL((index_score_mfma_kernel<HT, 1, 4>), grid, dim3(256), 0, stream, a, q, w, p.pools, scores); \
+        else                                                                                                        \
+            hipLaunchKernelGGL((index_score_mfma_kernel<HT, 8, 1>), grid, dim3(512), 0, stream, a, q, w, p.pools, scores); \
+    }
+                    AIGPU_IX(1) AIGPU_IX(2) AIGPU_IX(4)
+#undef AIGPU_IX
+                    return;
+                }
                 // about 2048 workgroups: a decode step splits its pools 256 ways,
                 // a long prefill gives each token one workgroup and one load of q
                 const uint64_t blocks = (maxPools + IX_POOLS - 1) / IX_POOLS;

@@ -136,3 +136,59 @@ def test_rejects_bad_shapes(gpu):
 def test_more_than_8192_pools_per_token(gpu):
     """past 256 x 32 pools a token's scores are streamed rather than held in registers"""
     run(gpu, 3, 8300, pool=1, top_k=64, heads=2, dim=32)
+
+
+@pytest.mark.parametrize("count,heads,dim", [(70, 48, 128), (40, 20, 100), (9, 7, 64), (17, 16, 36), (3, 64, 128),
+                                             (33, 16, 256)])
+def test_score_tiles(gpu, count, heads, dim):
+    """heads and dim short of the matrix-core kernel's tiles of 16 and 32, one to
+    four tokens a wave, token groups cut short, both ways of sharing a block of
+    64 pools, and a dim past it (index_score_kernel); the last block of pools
+    is cut short too"""
+    run(gpu, count, 300, heads=heads, dim=dim, pool=2, top_k=16)
+
+
+@pytest.mark.parametrize("count", [2, 40])
+def test_scores_of_values_that_are_not_finite(gpu, count):
+    """an infinite or NaN channel in a pool, and an infinite query: every score
+    equals the fp32 sums' (relu of a NaN product is 0, infinities carry)"""
+    import torch
+    heads, dim, hidden, q_rank, pool, start = 4, 64, 64, 32, 1, 200
+    r = np.random.default_rng(9)
+    w = {n: r.standard_normal(s).astype(np.float32) for n, s in
+         (("k", (dim, hidden)), ("gate", (dim, hidden)), ("q", (heads * dim, q_rank)), ("w", (heads, hidden)))}
+    dev = {n: {"w": to_device(x), "kind": "f32", "out": x.shape[0], "in": x.shape[1], "scales": None}
+           for n, x in w.items()}
+    h, qr = (r.standard_normal((count, n)).astype(np.float32) for n in (hidden, q_rank))
+    qr[count - 1, 3] = np.inf   # the last token's queries: infinities of both signs
+    cap = start + count + 1
+    pools = r.standard_normal((cap + 1, dim)).astype(np.float32)
+    pools[5, 7], pools[70, 0], pools[131, 63] = np.inf, np.nan, -np.inf
+    d_pools = dev_f32(pools)
+    keys, gates = (torch.zeros((cap, dim), dtype=torch.float32, device="cuda") for _ in range(2))
+    i32 = dict(dtype=torch.int32, device="cuda")
+    scores = torch.zeros((count, start + count), dtype=torch.float32, device="cuda")
+    say("select keys, not finite", dict(count=count))
+    gpu.select_keys(dev_f32(h), dev_f32(qr), dev, dev_f32(np.ones(dim)), None, dev_f32(np.zeros((1, dim))), keys, gates,
+                    d_pools, torch.zeros(count, **i32), torch.zeros(count, **i32), torch.zeros(count * 9, **i32), start,
+                    heads, dim, 8, pool, scores=scores)
+    got, p = host(scores), host(d_pools)
+    with np.errstate(all="ignore"):
+        q = np.stack([sum(qr[:, [j]] * w["q"][:, j][None] for j in range(q_rank))])[0].reshape(count, heads, dim)
+        wt = h @ w["w"].T / np.sqrt(heads)
+        for t in range(count):
+            n = start + t + 1
+            logit = np.zeros((heads, n), np.float32)
+            for d in range(dim):   # plain sums: an infinity or a NaN anywhere shows as it does in any order
+                logit += q[t][:, [d]] * p[None, :n, d]
+            logit /= np.sqrt(dim)
+            want = sum(wt[t, i] * np.where(logit[i] > 0, logit[i], 0) for i in range(heads))
+            bad = ~np.isfinite(want)
+            assert bad.any() and (np.isnan(got[t, :n]) == np.isnan(want)).all(), f"token {t}"
+            inf = np.isinf(want)
+            np.testing.assert_array_equal(got[t, :n][inf], want[inf])
+            # finite scores: fp32 sums of dim products per head; those of a row that is not finite are sums of
+            # relu(NaN) = relu(-inf) = 0 and so 0 themselves
+            tol = 1e-4 * (np.abs(wt[t])[:, None] * (np.abs(q[t]) @ np.abs(p[:n]).T)).sum(0) + 1e-6
+            tol = np.where(np.isfinite(tol), tol, 0.0)
+            assert (np.abs(got[t, :n] - want)[~bad] <= tol[~bad]).all()
