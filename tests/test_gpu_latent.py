@@ -84,3 +84,33 @@ def test_rejects_bad_rank(gpu):
     out = torch.zeros((1, 2, 8), device="cuda")
     with pytest.raises(RuntimeError, match="kvLoraRank"):
         gpu.latent_attention(q, lat, w, out, 0, 1.0)
+
+
+@pytest.mark.parametrize("count,start,heads,dn,dv,C,bf16", [
+    (1, 0, 1, 1, 1, 16, False), (1, 15, 16, 9, 65, 272, True), (1, 16, 17, 64, 128, 512, True),
+    (1, 31, 33, 128, 130, 496, False), (1, 32, 128, 192, 256, 512, True), (1, 4200, 40, 32, 24, 512, False),
+    (9, 63, 18, 200, 72, 400, True), (2, 64, 16, 256, 256, 512, False)])
+def test_tiles(gpu, count, start, heads, dn, dv, C, bf16):
+    """16 and 32 heads a workgroup with heads left over, splits of one to several
+    blocks of 32 keys whose last holds 1, 16, 17 or all of its keys, ranks past
+    one 256-column piece and short of two, v rows past one workgroup's 64"""
+    run(gpu, count, start, heads, dn, dv, C, 11, bf16_w=bf16)
+
+
+def test_kv_b_off_16_byte_boundaries(gpu):
+    """kv_b_proj 8 bytes past a 16-byte boundary: its rows are read 16 bytes at a time all the same"""
+    import torch
+    r = np.random.default_rng(12)
+    heads, dn, dv, C, start = 18, 40, 33, 64, 70
+    q, latent = (r.standard_normal(s).astype(np.float32) for s in ((1, heads, dn), (start + 1, C)))
+    bits = O.pack_bf16((r.standard_normal((heads * (dn + dv), C)) / 8).astype(np.float32)).reshape(-1, C)
+    wkv = O.unpack_bf16(bits).reshape(bits.shape)
+    store = torch.zeros(bits.size + 4, dtype=torch.bfloat16, device="cuda")
+    dw = store[4:].view(bits.shape)
+    dw.copy_(dev_bf16(bits))
+    assert dw.data_ptr() % 16 == 8
+    out = torch.zeros((1, heads, dv), dtype=torch.float32, device="cuda")
+    say("latent attention, kv_b off 16 bytes", {})
+    gpu.latent_attention(dev_f32(q), dev_f32(latent), dw, out, start, 0.125)
+    want = O.latent_attention(q, latent, wkv, start, heads, dn, dv, 0.125)
+    assert np.abs(host(out) - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
