@@ -107,14 +107,25 @@ __device__ __forceinline__ void lower_block(int b, int& I, int& J) {
 }
 
 /*
-    Per (value head, chunk), 256 threads. LDS (KD 128): kn, qn, gc
-    [64][KD+4] and Am, Qm, Tm [64][68], about 155 KB.
+    Per (value head, chunk), KD / 8 waves: the LDS (KD 128: kn, qn, gc
+    [64][KD+4] and Am, Qm, Tm [64][68], about 155 KB) holds one workgroup a CU,
+    so its own waves must cover each other's LDS reads and exps (four per SIMD
+    at KD 128). In the two pairs of products at the end a wave has one
+    16-column tile, whose column operand is read once and stays in registers,
+    and the rows of Tb and P come as 16-byte reads (k slot of step s: 16 M + 4 g
+    + s). Bound by its chain of short phases (a quarter of its cycles have an
+    MFMA running): 2,048 workgroups (4,096 tokens, 32 heads of 128) 220 us, 235
+    with eight waves, 305 with four and scalar operand reads.
 */
+template <int KD> constexpr int solve_threads() { return 8 * KD; }
+
 template <int KD, bool F32>
-__global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
+__global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs a) {
+    constexpr int SOLVE_THREADS = solve_threads<KD>(), WAVES = SOLVE_THREADS / 64;
     constexpr int KS = KD + 4;
-    constexpr int PE = KD / 4;   // row elements per thread in the row passes
-    constexpr int VPRE = CH * KD / 8 / 256;   // 8-element value pieces per thread per slab
+    constexpr int TR = SOLVE_THREADS / CH;   // threads per row in the row passes
+    constexpr int PE = KD / TR;              // row elements of each
+    constexpr int VPRE = CH * KD / 8 / SOLVE_THREADS;   // 8-element value pieces per thread per slab
     __shared__ __align__(16) float kn[CH * KS];
     __shared__ __align__(16) float qn[CH * KS];
     __shared__ __align__(16) float gc[CH * KS];   // log2 decays; later the value slabs
@@ -136,7 +147,7 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     // ---- q, k rows normalised (LocalModel.hpp:1380-1386, q also scaled by
     //      1/sqrt(KD) as :2935); log2 decays; beta. Rows past the end are zero.
     {
-        const int r = tid >> 2, qq = tid & 3;
+        const int r = tid / TR, qq = tid % TR;
         const bool live = uint32_t(r) < n;
         const uint64_t tr = t0 + (live ? r : 0);
         float kx[PE], qx[PE];
@@ -148,10 +159,11 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
             kss = fmaf(kx[e], kx[e], kss);
             qss = fmaf(qx[e], qx[e], qss);
         }
-        kss += __shfl_xor(kss, 1, WAVE);
-        kss += __shfl_xor(kss, 2, WAVE);
-        qss += __shfl_xor(qss, 1, WAVE);
-        qss += __shfl_xor(qss, 2, WAVE);
+#pragma unroll
+        for (int o = 1; o < TR; o <<= 1) {
+            kss += __shfl_xor(kss, o, WAVE);
+            qss += __shfl_xor(qss, o, WAVE);
+        }
         float kinv = 1.0f, qinv = 1.0f;
         if (p.normalize) {
             kinv = 1.0f / sqrtf(kss + 1e-6f);
@@ -198,7 +210,7 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     const int sw0 = int(VD < size_t(KD) ? VD : KD);
     float vpre[VPRE][8];
     auto vload = [&](size_t c0, int sw, int it, float (&x)[8]) {
-        const int idx = tid + 256 * it;
+        const int idx = tid + SOLVE_THREADS * it;
         const int t = idx / (sw / 8), c = 8 * (idx % (sw / 8));
         if (idx < CH * (sw / 8) && uint32_t(t) < n) {
             load_row<F32, 8>(p.v, ((t0 + t) * Hv + h) * VD + c0 + c, x);
@@ -208,7 +220,7 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
         }
     };
     auto vstore = [&](int sw, int it, const float (&x)[8]) {
-        const int idx = tid + 256 * it;
+        const int idx = tid + SOLVE_THREADS * it;
         if (idx < CH * (sw / 8)) {
             const int t = idx / (sw / 8), c = 8 * (idx % (sw / 8));
             *reinterpret_cast<floatx4*>(&gc[t * KS + c]) = floatx4{x[0], x[1], x[2], x[3]};
@@ -220,9 +232,9 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     __syncthreads();
 
     // ---- cumulative log2 decay of each channel down the chunk: the rows in
-    //      256 / KD parts, each summed by its own thread, then offset ----
+    //      eight parts, each summed by its own thread, then offset ----
     {
-        constexpr int PARTS = 256 / KD, RPP = CH / PARTS;
+        constexpr int PARTS = SOLVE_THREADS / KD, RPP = CH / PARTS;
         const int ch = tid % KD, part = tid / KD;
         float col[RPP];
 #pragma unroll
@@ -239,8 +251,8 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     }
     __syncthreads();
 
-    // ---- the ten lower blocks of A and QKm: wave w takes blocks w, w+4, w+8 ----
-    for (int b = w; b < 10; b += 4) {
+    // ---- the ten lower blocks of A and QKm: a block per wave and turn ----
+    for (int b = w; b < 10; b += WAVES) {
         int I, J;
         lower_block(b, I, J);
         const int r0 = 16 * I, j0 = 16 * J;
@@ -301,7 +313,7 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
 
     // ---- T = (I + A)^-1 (lower blocks only): diagonal blocks by forward
     //      substitution in registers, then the block rows below on MFMA ----
-    {
+    if (w < 4) {
         const int b0 = 16 * w, j = lane & 15;
         float t[16];
 #pragma unroll
@@ -339,24 +351,24 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     __syncthreads();
 
     // ---- Tb = T diag(beta), in place ----
-    for (int idx = tid; idx < CH * CH; idx += 256) {
+    for (int idx = tid; idx < CH * CH; idx += SOLVE_THREADS) {
         const int t = idx / CH, j = idx % CH;
         if ((j >> 4) <= (t >> 4)) Tm[t * CS + j] *= bet[j];
     }
     __syncthreads();
 
-    // ---- P = QKm Tb into Am: wave w takes block row I = w ----
-    {
-        const int I = w;
-        for (int J = 0; J <= I; ++J) {
-            floatx4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int M = J; M <= I; ++M)
+    // ---- P = QKm Tb into Am: a block per wave and turn ----
+    for (int b = w; b < 10; b += WAVES) {
+        int I, J;
+        lower_block(b, I, J);
+        floatx4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int M = J; M <= I; ++M) {
+            const floatx4 qm = *reinterpret_cast<const floatx4*>(&Qm[(16 * I + c16) * CS + 16 * M + 4 * g]);
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    x = mfma4(Qm[(16 * I + c16) * CS + 16 * M + 4 * s + g], Tm[(16 * M + 4 * s + g) * CS + 16 * J + c16], x);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) Am[(16 * I + 4 * g + r) * CS + 16 * J + c16] = x[r];
+            for (int s = 0; s < 4; ++s) x = mfma4(qm[s], Tm[(16 * M + 4 * g + s) * CS + 16 * J + c16], x);
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Am[(16 * I + 4 * g + r) * CS + 16 * J + c16] = x[r];
     }
 
     // ---- the record: Kt and exp(gc_last) straight from kn, gc ----
@@ -366,7 +378,7 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     float* rK = rec + 2 * CH * KD;
     float* rE = rec + 3 * CH * KD;
     float* rUO = rE + KD;
-    for (int idx = tid; idx < CH * KD / 4; idx += 256) {
+    for (int idx = tid; idx < CH * KD / 4; idx += SOLVE_THREADS) {
         const int ln = idx % 64, q = (idx / 64) % (CH / 16), mt = idx / 64 / (CH / 16);
         const int m = 16 * mt + (ln & 15), j0 = 16 * q + 4 * (ln >> 4);
         const float gl = gc[(CH - 1) * KS + m];
@@ -378,7 +390,7 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     if (tid < KD) rE[tid] = exp2_fast(gc[(CH - 1) * KS + tid]);
     __syncthreads();
     // Kg, Qg in place
-    for (int idx = tid; idx < CH * KD / 4; idx += 256) {
+    for (int idx = tid; idx < CH * KD / 4; idx += SOLVE_THREADS) {
         const int t = idx / (KD / 4), i = 4 * (idx % (KD / 4));
         const floatx4 gv = *reinterpret_cast<const floatx4*>(&gc[t * KS + i]);
         floatx4 kv = *reinterpret_cast<floatx4*>(&kn[t * KS + i]);
@@ -394,25 +406,34 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
     }
     __syncthreads();
 
-    // Block row I of Tb and of P has I + 1 nonzero blocks: waves 0, 1 take
-    // rows 0 and 3, waves 2, 3 rows 1 and 2, each half of the column tiles.
-    const int rowA = (w < 2) ? 0 : 1, rowB = 3 - rowA, par = w & 1;
+    // Two waves share a 16-column tile c: block row I has I + 1 nonzero blocks,
+    // so one takes rows 0 and 3, the other rows 1 and 2 (KD / 16 tiles at most)
+    auto ld4 = [](const float* ptr) { return *reinterpret_cast<const floatx4*>(ptr); };
+    const int c = w % (KD / 16), second = w / (KD / 16);
 
     // ---- -W = -Tb Kg and Qt = Qg - P Kg, computed transposed (key rows,
     //      token columns) so each lane's accumulator is one scan fragment ----
-    for (int pass = 0; pass < 2; ++pass) {
-        const int I = pass ? rowB : rowA;
-        for (int c = par; c < KD / 16; c += 2) {
+    {
+        float ak[4][4];   // Kg[16 M + 4 g + s][16 c + c16]
+#pragma unroll
+        for (int M = 0; M < 4; ++M)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) ak[M][s] = kn[(16 * M + 4 * g + s) * KS + 16 * c + c16];
+#pragma unroll
+        for (int I = 0; I < 4; ++I) {
+            if (second != ((I == 0 || I == 3) ? 0 : 1)) continue;   // uniform
             floatx4 xw = {0.0f, 0.0f, 0.0f, 0.0f};
-            floatx4 xq = *reinterpret_cast<const floatx4*>(&qn[(16 * I + c16) * KS + 16 * c + 4 * g]);
-            for (int M = 0; M <= I; ++M)
+            floatx4 xq = ld4(&qn[(16 * I + c16) * KS + 16 * c + 4 * g]);
+#pragma unroll
+            for (int M = 0; M <= I; ++M) {
+                const floatx4 tm = ld4(&Tm[(16 * I + c16) * CS + 16 * M + 4 * g]);
+                const floatx4 pm = ld4(&Am[(16 * I + c16) * CS + 16 * M + 4 * g]);
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const int k = 16 * M + 4 * s + g;
-                    const float ak = kn[k * KS + 16 * c + c16];
-                    xw = mfma4(ak, -Tm[(16 * I + c16) * CS + k], xw);
-                    xq = mfma4(ak, -Am[(16 * I + c16) * CS + k], xq);
+                    xw = mfma4(ak[M][s], -tm[s], xw);
+                    xq = mfma4(ak[M][s], -pm[s], xq);
                 }
+            }
             const int frag = (I * (KD / 16) + c) * 64 + lane;
             reinterpret_cast<floatx4*>(rW)[frag] = xw;
             reinterpret_cast<floatx4*>(rQ)[frag] = xq;
@@ -434,19 +455,27 @@ __global__ __launch_bounds__(256) void kda_solve_kernel(KdaArgs a) {
             }
         }
         __syncthreads();
-        for (int pass = 0; pass < 2; ++pass) {
-            const int I = pass ? rowB : rowA;
-            for (int c = par; c < sw / 16; c += 2) {
+        if (c < sw / 16) {
+            float bv[4][4];   // V[16 M + 4 g + s][16 c + c16]
+#pragma unroll
+            for (int M = 0; M < 4; ++M)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) bv[M][s] = gc[(16 * M + 4 * g + s) * KS + 16 * c + c16];
+            floatx4* blk = reinterpret_cast<floatx4*>(rUO + (c0 / 16 + c) * (2 * CH * 16));
+#pragma unroll
+            for (int I = 0; I < 4; ++I) {
+                if (second != ((I == 0 || I == 3) ? 0 : 1)) continue;   // uniform
                 floatx4 xu = {0.0f, 0.0f, 0.0f, 0.0f}, xo = {0.0f, 0.0f, 0.0f, 0.0f};
-                for (int M = 0; M <= I; ++M)
+#pragma unroll
+                for (int M = 0; M <= I; ++M) {
+                    const floatx4 tm = ld4(&Tm[(16 * I + c16) * CS + 16 * M + 4 * g]);
+                    const floatx4 pm = ld4(&Am[(16 * I + c16) * CS + 16 * M + 4 * g]);
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
-                        const int k = 16 * M + 4 * s + g;
-                        const float bv = gc[k * KS + 16 * c + c16];
-                        xu = mfma4(Tm[(16 * I + c16) * CS + k], bv, xu);
-                        xo = mfma4(Am[(16 * I + c16) * CS + k], bv, xo);
+                        xu = mfma4(tm[s], bv[M][s], xu);
+                        xo = mfma4(pm[s], bv[M][s], xo);
                     }
-                floatx4* blk = reinterpret_cast<floatx4*>(rUO + (c0 / 16 + c) * (2 * CH * 16));
+                }
                 blk[I * 64 + lane] = xu;
                 blk[(CH / 16 + I) * 64 + lane] = xo;
             }
@@ -600,7 +629,7 @@ bool launch_kda(const KdaParams& p, hipStream_t stream) {
 #define AIGPU_KDA(KD, F)                                                                                       \
     if (p.keyDim == KD && (p.inType == 0) == F) {                                                              \
         if (!ctx.launch("kda_solve_kernel", stream, [&] {                                                      \
-                hipLaunchKernelGGL((kda_solve_kernel<KD, F>), sgrid, dim3(256), 0, stream, a);                 \
+                hipLaunchKernelGGL((kda_solve_kernel<KD, F>), sgrid, dim3(solve_threads<KD>()), 0, stream, a);                 \
             }))                                                                                                \
             return false;                                                                                      \
         return ctx.launch("kda_scan_kernel", stream, [&] {                                                     \
