@@ -144,3 +144,10 @@ def test_rejects_mismatched_shapes(gpu):
     gpu.prefill_mixer(x, w, out, kc, kc, 0, 2, 2, 128)   # 2 heads of 128: every shape fits
     with pytest.raises(RuntimeError, match="weight shapes"):   # 4 heads: q needs 512 rows
         gpu.prefill_mixer(x, w, out, kc, kc, 0, 4, 2, 128)
+
+
+@pytest.mark.parametrize("kind,gate", [("bf16", False), ("q8", True)])
+def test_key_splits_behind_a_history(gpu, kind, gate):
+    """few rows behind 1500 positions: the attention's keys are split, and the merge writes the o projection's operand
+    images"""
+    run(gpu, kind, count=20, start=1500, gate=gate)

@@ -170,3 +170,19 @@ def test_output_gate_needs_wide_rows(gpu):
     import aigpu
     with pytest.raises(aigpu.AiGpuError, match="output gate"):
         run_case(gpu, 4, 0, 2, 1, 64, 78, q_stride=64, gate=True)
+
+
+@pytest.mark.parametrize("count,start,H,KV,D,window,gate,dtype", [
+    (1, 1151, 8, 2, 128, 0, False, "bf16"),     # 9 tiles in three splits, one row
+    (257, 640, 16, 8, 128, 0, False, "f32"),    # two query tiles, the second of one row; a split of it alone empty
+    (40, 2000, 4, 4, 128, 129, True, "bf16"),   # a window that leaves whole splits out of sight, the gate in the merge
+    (333, 1500, 8, 2, 64, 0, True, "bf16"), (20, 3000, 8, 8, 64, 1000, False, "f32"),
+    (90, 1100, 6, 3, 128, 0, False, "bf16")])   # a grid that does not divide over the XCDs
+def test_key_splits_behind_a_history(gpu, count, start, H, KV, D, window, gate, dtype):
+    """a short call behind a history splits its keys over the idle CUs
+    (prefill_merge_kernel combines them), and its prep's extra workgroups
+    convert the history"""
+    ref, got, kn, v, kc, vcb, vb = run_case(gpu, count, start, H, KV, D, 70 + count, window=window, gate=gate,
+                                            dtype=dtype, q_stride=2 * D if gate else None)
+    assert_bf16_parity(ref, got, f"splits {count} after {start}")
+    assert np.abs(kc[:, start:start + count].transpose(1, 0, 2) - kn).max() <= np.abs(kn).max() * 2 ** -8
