@@ -983,16 +983,16 @@ def cfg1_workload(args, cpu):
     def step():
         aigpu.attention_device(qf, kf, vf, of, S, 0, H, H, D, D, H * D, D)
 
-    step_ms, k_ms, launched_ms = time_steps(step, max(args.steps, 50), args.warmup, "attention_f32_tile_kernel")
+    step_ms, k_ms, launched_ms = time_steps(step, max(args.steps, 50), args.warmup, "attention_f32_narrow_kernel")
     flops = 4.0 * D * H * S * (S + 1) / 2
     res = {"workload": "configs[0] gpt2-small MHA prefill fp32 S=128 12 heads D=64", "dtype": "f32",
            "unit": "TFLOP/s", "value": flops / (step_ms * 1e-3) / 1e12, "ms_per_step": step_ms,
-           "roofline": {"kernel": "attention_f32_tile_kernel", "bound": "fp32",
+           "roofline": {"kernel": "attention_f32_narrow_kernel", "bound": "fp32",
                         "achieved": flops / (k_ms * 1e-3) / 1e12, "peak": PEAK_MFMA_F32, "unit": "TFLOP/s",
                         "frac": flops / (k_ms * 1e-3) / 1e12 / PEAK_MFMA_F32, "traffic": None, "kernel_ms": k_ms,
                         "flops_per_launch": flops, "kernels_ms_per_step": launched_ms,
                         "note": "latency-bound: 25.4 MFLOP take 0.16 us at the fp32 peak; the step is the "
-                                "tiled kernel (keys split in two) and the merge of its records"}}
+                                "narrow kernel alone (16 query rows a workgroup, keys over its waves)"}}
     if cpu is not None:
         O, ref, kind, threads = cpu
         qh, kh, vh = (np.ascontiguousarray(t.cpu().numpy()) for t in (qf, kf, vf))
@@ -1043,7 +1043,7 @@ def published_workload(args, cpu):
     def step_f32():
         aigpu.attention_device(q, keys, vals, out, n, start, H, KV, D, D, KV * D, D)
 
-    f_ms, fk_ms, f_all = time_steps(step_f32, max(args.steps, 50), args.warmup, "attention_f32_tile_kernel")
+    f_ms, fk_ms, f_all = time_steps(step_f32, max(args.steps, 50), args.warmup, "attention_f32_narrow_kernel")
     got_f32 = out.cpu().numpy()
     # the bf16 flash path: history in the head-major bf16 cache, the 128 new
     # rows through prep (no norm, no RoPE: kernels::attention alone)

@@ -4,9 +4,10 @@
 // first = start+t+1-window when a window is set; out = softmax(q.K/sqrt(D)) V.
 //
 // This is the exact-arithmetic path behind the drop-in aigpu_attention, in
-// two forms. fp32 q and KV of dim 64 or 128 on 16-byte boundaries take the
-// tiled form on the fp32 matrix cores (attention_f32_tile_kernel, described
-// at it); every other call (bf16 KV, other dims, unaligned rows) takes the
+// these forms. fp32 q and KV of dim 64 or 128 on 16-byte boundaries take the
+// fp32 matrix cores, in tiles of 128 tokens or, where those leave the chip
+// idle, in groups of 16 query rows (attention_f32_tile_kernel and
+// attention_f32_narrow_kernel, described at them); every other call (bf16 KV, other dims, unaligned rows) takes the
 // scalar form: fp32 loads, fp32 FMAs, expf. There one wave owns one (token,
 // head) and walks the keys in blocks of 64 with an online softmax: lane j
 // scores key j of the block, then the lanes switch to owning dimensions for
@@ -238,9 +239,9 @@ struct TileArgs {
     AttentionF32Params p;
     float* acc;              // split records [split][head][token][dim]
     float2* ml;              // their (m, l) [split][head][token]
-    uint32_t groups;         // token groups of TQ
-    uint32_t splits;         // workgroups per (token group, head)
-    uint32_t tilesPerSplit;  // key tiles per workgroup when splits > 1
+    uint32_t groups;         // token groups of TQ (narrow: row groups of NR)
+    uint32_t splits;         // workgroups per (token group, head) (narrow: per (row group, kv head))
+    uint32_t tilesPerSplit;  // key tiles per workgroup when splits > 1; 0: the narrow form
 };
 
 /* the key tiles of token group `grp`: every key a token of the group sees
@@ -479,6 +480,188 @@ __global__ __launch_bounds__(256) void attention_f32_tile_kernel(TileArgs a) {
     if (h == 0) a.ml[rec] = make_float2(m, lsum);
 }
 
+/*
+    The narrow form, for calls whose tiles of 128 tokens would leave most of
+    the chip idle: a workgroup owns 16 query rows of one kv head (a row is a
+    (token, query head) pair, token-major, so a group's heads share the K and
+    V they read) and its NW waves take 16-key blocks in turn, each with its
+    own softmax state, combined in LDS at the end. K, V and q go from memory
+    to the operand registers 16 bytes a lane, a block ahead of its products:
+    nothing is shared between waves, so there is nothing to stage.
+
+    S^T (16 keys x 16 rows) = K Q^T on v_mfma_f32_16x16x4_f32: lane group g
+    (lane / 16) supplies dims g D/4 + s at step s, so a lane reads D/4
+    contiguous floats of key lane % 16. Register r of the block is key
+    4 g + r for row lane % 16, which is the B operand of P.V's step r; its A
+    operand, row i of d tile dt, is dim i D/16 + dt, so a lane reads D/16
+    contiguous floats of that key's value, and O^T leaves it D/4 contiguous
+    dims of its row.
+
+    A row that saw only scores of -inf keeps m = -inf with l = 0; NaN scores
+    stay NaN in l and o, whatever m is.
+*/
+constexpr int NR = 16;     // query rows per workgroup
+constexpr int NB = 16;     // keys per block
+constexpr int NW = 8;      // waves per workgroup
+
+template <int D>
+__global__ __launch_bounds__(64 * NW, D == 64 ? 4 : 2) void attention_f32_narrow_kernel(TileArgs a) {
+    constexpr int KF = D / 16;             // 16-byte K (and q) pieces per lane
+    constexpr int VF = D / 64;             // 16-byte V pieces per lane and key
+    constexpr int DT = D / 16;             // 16-dim tiles of O^T
+    constexpr int OS = D + 4;              // floats per row of Os
+    __shared__ __attribute__((aligned(16))) float Os[NW * NR * OS];
+    __shared__ float2 Ml[NW][NR];
+
+    const AttentionF32Params& p = a.p;
+    const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(uint32_t(threadIdx.x >> 6));
+    // 32 bits hold every row, position and block here (launch_tiled)
+    const uint32_t heads = uint32_t(p.heads), kvHeads = uint32_t(p.kvHeads), G = heads / kvHeads;
+    const uint32_t count = uint32_t(p.count), start = uint32_t(p.start), rows = count * G;
+    uint32_t bid = blockIdx.x;
+    const uint32_t sigma = bid % a.splits;
+    bid /= a.splits;
+    const uint32_t kv = bid % kvHeads, grp = a.groups - 1 - bid / kvHeads;   // the longest groups first
+    const uint32_t row0 = grp * NR, rowLast = row0 + NR < rows ? row0 + NR - 1 : rows - 1;
+    auto firstKey = [&](uint32_t pos) __attribute__((always_inline)) {
+        return p.window && pos + 1 > p.window ? pos + 1 - uint32_t(p.window) : 0u;
+    };
+    // keys any row sees: [kbeg, kend)
+    const uint32_t kbeg = firstKey(start + row0 / G), kend = start + rowLast / G + 1;
+    const uint32_t nb = (kend - kbeg + NB - 1) / NB;
+    const uint32_t bBegin = uint32_t(uint64_t(nb) * sigma / a.splits), bEnd = uint32_t(uint64_t(nb) * (sigma + 1) / a.splits);
+
+    // rows past the last repeat it and store nothing
+    const uint32_t row = row0 + j < rows ? row0 + j : rows - 1, t = row / G, head = kv * G + row % G;
+    const uint32_t P = start + t, first = firstKey(P);
+    const float* kbase = static_cast<const float*>(p.keys) + kv * p.headStride + g * (D / 4);
+    const float* vbase = static_cast<const float*>(p.values) + kv * p.headStride + j * (D / 16);
+    const uint32_t posStride = uint32_t(p.posStride);
+
+    floatx4 qf[KF];
+    {
+        const float* qrow = static_cast<const float*>(p.q) + (uint64_t(t) * heads + head) * p.qStride + g * (D / 4);
+#pragma unroll
+        for (int i = 0; i < KF; ++i)
+            qf[i] = *reinterpret_cast<const floatx4*>(qrow + 4 * i);
+    }
+    // keys past the group's last repeat it (their scores are masked, their P is 0)
+    auto load = [&](uint32_t b, floatx4 (&kf)[KF], floatx4 (&vf)[4][VF]) __attribute__((always_inline)) {
+        const uint32_t k0 = kbeg + b * NB;
+        const float* kr = kbase + uint64_t(k0 + j < kend ? k0 + j : kend - 1) * posStride;
+#pragma unroll
+        for (int i = 0; i < KF; ++i) kf[i] = *reinterpret_cast<const floatx4*>(kr + 4 * i);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t vk = k0 + 4 * g + r;
+            const float* vr = vbase + uint64_t(vk < kend ? vk : kend - 1) * posStride;
+#pragma unroll
+            for (int i = 0; i < VF; ++i) vf[r][i] = *reinterpret_cast<const floatx4*>(vr + 4 * i);
+        }
+    };
+
+    floatx4 o[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    float m = -INFINITY, lsum = 0.0f;
+    const float scale = 1.0f / sqrtf(float(D));
+
+    floatx4 kf[KF], vf[4][VF];
+    if (bBegin + w < bEnd) load(bBegin + w, kf, vf);
+    for (uint32_t b = bBegin + w; b < bEnd; b += NW) {
+        floatx4 kn[KF], vn[4][VF];
+        if (b + NW < bEnd) load(b + NW, kn, vn);
+        floatx4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < KF; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i][e], qf[i][e], s, 0, 0, 0);
+        const uint32_t k0 = kbeg + b * NB + 4 * g;
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = k0 + r >= first && k0 + r <= P ? s[r] * scale : -INFINITY;
+            mx = fmaxf(mx, s[r]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        const float mn = fmaxf(m, mx), mz = mn == -INFINITY ? 0.0f : mn;   // all -inf so far: zeros (or NaN)
+        const float alpha = expf(m - mz);
+        float psum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[r] = expf(s[r] - mz);
+            psum += s[r];
+        }
+        psum += __shfl_xor(psum, 16, WAVE);
+        psum += __shfl_xor(psum, 32, WAVE);
+        lsum = lsum * alpha + psum;
+        m = mn;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[r][dt / 4][dt % 4], s[r], o[dt], 0, 0, 0);
+        if (b + NW < bEnd) {
+#pragma unroll
+            for (int i = 0; i < KF; ++i) kf[i] = kn[i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int i = 0; i < VF; ++i) vf[r][i] = vn[r][i];
+        }
+    }
+
+    // O^T register r of d tile dt is dim (4 g + r) D/16 + dt: a lane's D/4
+    // dims from g D/4 on, in the order (r, dt)
+    float* ow = Os + (w * NR + j) * OS + g * (D / 4);
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) {
+        floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = o[(4 * i + e) % DT][(4 * i + e) / DT];
+        *reinterpret_cast<floatx4*>(ow + 4 * i) = v;
+    }
+    if (g == 0) Ml[w][j] = make_float2(m, lsum);
+    __syncthreads();
+
+    // one 16-byte piece of a row per thread; a wave without a block left m =
+    // -inf with zeros, and m = -inf weighs 0 (its l and o are zeros, or NaN)
+    constexpr int PIECES = D / 4;
+    const uint32_t r = threadIdx.x / PIECES, c = threadIdx.x % PIECES;
+    if (r >= NR || row0 + r >= rows) return;
+    const uint32_t ot = (row0 + r) / G, oh = kv * G + (row0 + r) % G;
+    float M = -INFINITY, L = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NW; ++u) M = fmaxf(M, Ml[u][r].x);
+    const float Mz = M == -INFINITY ? 0.0f : M;
+    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < NW; ++u) {
+        const float2 ml = Ml[u][r];
+        const float e = expf(ml.x - Mz);
+        const floatx4 v = *reinterpret_cast<const floatx4*>(Os + (u * NR + r) * OS + 4 * c);
+        L += ml.y * e;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += v[i] * e;
+    }
+    if (a.splits == 1) {
+        const float inv = 1.0f / L;
+        *reinterpret_cast<floatx4*>(p.out + (uint64_t(ot) * heads + oh) * D + 4 * c) =
+            floatx4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+        return;
+    }
+    const size_t rec = (size_t(sigma) * heads + oh) * count + ot;
+    *reinterpret_cast<floatx4*>(a.acc + rec * D + 4 * c) = acc;
+    // the merge leaves out records of m = -inf: one that holds NaN keeps it
+    if (c == 0) a.ml[rec] = make_float2(M == -INFINITY && L != L ? 0.0f : M, L);
+}
+
 /* one wave per (token, head): out = sum_s e^(m_s - M) o_s / sum_s e^(m_s - M) l_s
    over the splits that cover the token's group (a split in which the row
    saw no key has m = -inf and adds nothing); the records of up to MB splits
@@ -491,10 +674,13 @@ __global__ __launch_bounds__(256) void attention_f32_merge_kernel(TileArgs a) {
     const uint64_t task = uint64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
     if (task >= p.count * p.heads) return;
     const uint64_t t = task / p.heads, head = task % p.heads;
-    uint64_t kbeg;
-    uint32_t ntiles;
-    group_tiles(p.count, p.start, p.window, t / TQ, kbeg, ntiles);
-    const uint32_t n = (ntiles + a.tilesPerSplit - 1) / a.tilesPerSplit;
+    uint32_t n = a.splits;           // the narrow form's splits all leave a record
+    if (a.tilesPerSplit) {
+        uint64_t kbeg;
+        uint32_t ntiles;
+        group_tiles(p.count, p.start, p.window, t / TQ, kbeg, ntiles);
+        n = (ntiles + a.tilesPerSplit - 1) / a.tilesPerSplit;
+    }
     float M = -INFINITY, L = 0.0f, acc[NE] = {};
     for (uint32_t s0 = 0; s0 < n; s0 += MB) {
         float2 ml[MB];
@@ -541,6 +727,91 @@ bool tile_eligible(const AttentionF32Params& p) {
            p.headStride % 4 == 0 && p.posStride < (uint64_t(1) << 22);
 }
 
+/* room for a.splits records of every row */
+bool split_records(TileArgs& a) {
+    const AttentionF32Params& p = a.p;
+    const size_t accBytes = size_t(a.splits) * p.heads * p.count * p.dim * 4;
+    char* parts = static_cast<char*>(
+        Context::instance().grow(SLOT_ATTN_PARTS, accBytes + size_t(a.splits) * p.heads * p.count * 8));
+    if (!parts) return false;
+    a.acc = reinterpret_cast<float*>(parts);
+    a.ml = reinterpret_cast<float2*>(parts + accBytes);
+    return true;
+}
+
+bool launch_merge(const TileArgs& a, hipStream_t stream) {
+    const bool d64 = a.p.dim == 64;
+    const uint64_t mblocks = (a.p.count * a.p.heads + 3) / 4;
+    return Context::instance().launch("attention_f32_merge_kernel", stream, [&] {
+        if (d64) hipLaunchKernelGGL(attention_f32_merge_kernel<64>, dim3(unsigned(mblocks)), dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL(attention_f32_merge_kernel<128>, dim3(unsigned(mblocks)), dim3(256), 0, stream, a);
+    });
+}
+
+/*
+    Tiled or narrow, and the narrow form's splits: by the modelled time (us)
+    of each. A workgroup's serial chain sets both: `rounds` workgroups per
+    CU, each walking its longest key range. A tile of 64 keys x 128 tokens
+    takes 9 us of a CU at dim 128 (two workgroups of dim 64 share one); a
+    narrow step, a block of 16 keys in each of NW waves, 3.2 us at dim 128 and
+    1.5 at 64; a merge launch 2.8 to 3.8 us and its records. The constants
+    are fitted to 140 shapes, 1 to 512 tokens behind 0 to 2000 positions at
+    five head counts (7% rms); 8% closer than that, the tiled form keeps the
+    call. 128 tokens from empty at 12 x 64: 15.9 -> 10.3 us, at 32q/8kv x 128
+    24.3 -> 11.8; one token after 2000 at 32q/8kv x 128 48.5 -> 14.9; 64
+    tokens after 2000 62.5 -> 42.3. Where tiles fill the chip they read K and
+    V for eight times the rows: 256 tokens after 2000 at 32q/8kv x 128 take
+    108 us tiled, 118 narrow; 700 from empty at 64 x 128, window 256, 101 and
+    126.
+*/
+double merge_cost(bool d64, bool narrow, double recordBytes) {
+    return narrow ? 2.8 + recordBytes * (d64 ? 0.3e-6 : 1.2e-6) : 3.8 + recordBytes * 0.9e-6;
+}
+
+double rounds(uint64_t blocks, uint64_t slots) { return double((blocks + slots - 1) / slots); }
+
+/* the narrow form's splits for this call, or 0 where the tiled form's
+   `tiled` us are less */
+uint32_t narrow_splits(const AttentionF32Params& p, double tiled) {
+    // rows and positions in 32 bits
+    if (p.count >= (1u << 30) || p.start >= (1u << 30) || p.heads >= (1u << 20) ||
+        p.count * p.heads >= (uint64_t(1) << 30))
+        return 0;
+    const bool d64 = p.dim == 64;
+    const uint64_t G = p.heads / p.kvHeads, wgs = (p.count * G + NR - 1) / NR * p.kvHeads;
+    uint64_t keys = p.start + p.count;                       // the longest row group's
+    const uint64_t span = (NR + G - 1) / G;                  // tokens of a row group, less one
+    if (p.window && p.window + span < keys) keys = p.window + span;
+    const uint64_t nb = (keys + NB - 1) / NB;
+    const uint64_t rowBytes = p.count * p.heads * (p.dim * 4 + 8);
+    uint32_t best = 0;
+    for (uint32_t sp = 1; sp == 1 || (4 * sp <= nb && sp <= 64 && sp * rowBytes <= (uint64_t(256) << 20)); sp *= 2) {
+        const double steps = double((nb + uint64_t(NW) * sp - 1) / (uint64_t(NW) * sp));
+        const double us = 8.0 + rounds(wgs * sp, 256) * (d64 ? 1.5 * steps + 0.4 : 3.2 * steps) +
+                          (sp > 1 ? merge_cost(d64, true, double(sp * rowBytes)) : 0.0);
+        if (us < tiled) tiled = us, best = sp;
+    }
+    return best;
+}
+
+bool launch_narrow(TileArgs a, hipStream_t stream, uint32_t splits) {
+    Context& ctx = Context::instance();
+    const AttentionF32Params& p = a.p;
+    a.groups = uint32_t((p.count * (p.heads / p.kvHeads) + NR - 1) / NR);
+    a.splits = splits;
+    a.tilesPerSplit = 0;
+    if (a.splits > 1 && !split_records(a)) return false;
+    const uint64_t blocks = uint64_t(a.groups) * p.kvHeads * a.splits;
+    if (!ctx.launch("attention_f32_narrow_kernel", stream, [&] {
+            if (p.dim == 64)
+                hipLaunchKernelGGL(attention_f32_narrow_kernel<64>, dim3(unsigned(blocks)), dim3(64 * NW), 0, stream, a);
+            else
+                hipLaunchKernelGGL(attention_f32_narrow_kernel<128>, dim3(unsigned(blocks)), dim3(64 * NW), 0, stream, a);
+        }))
+        return false;
+    return a.splits == 1 || launch_merge(a, stream);
+}
+
 bool launch_tiled(const AttentionF32Params& p, hipStream_t stream) {
     Context& ctx = Context::instance();
     TileArgs a{};
@@ -566,27 +837,31 @@ bool launch_tiled(const AttentionF32Params& p, hipStream_t stream) {
     a.groups = uint32_t(groups);
     a.splits = tps < maxTiles ? uint32_t((maxTiles + tps - 1) / tps) : 1u;
     a.tilesPerSplit = a.splits > 1 ? uint32_t(tps) : maxTiles;
+    uint64_t live = 0;   // workgroups with tiles
+    for (uint64_t g = 0; g < groups; ++g) {
+        uint64_t kbeg;
+        uint32_t nt;
+        group_tiles(p.count, p.start, p.window, g, kbeg, nt);
+        live += (nt + a.tilesPerSplit - 1) / a.tilesPerSplit;
+    }
+    double tiles = rounds(live * p.heads, slots) * a.tilesPerSplit;
+    if (a.splits == 1) {   // ranges of all lengths, the longest first: they even out over the CUs
+        const double even = double(total) / double(slots) + 0.25 * maxTiles;
+        tiles = tiles < even ? tiles : even;
+    }
+    const double us = (p.dim == 64 ? 2.0 : 7.0) + 9.0 * tiles +
+                      (a.splits > 1 ? merge_cost(p.dim == 64, false, double(a.splits * perSplit)) : 0.0);
+    if (const uint32_t sp = narrow_splits(p, 0.92 * us)) return launch_narrow(a, stream, sp);
     const uint64_t blocks = groups * p.heads * a.splits;
     if (blocks > 0x7FFFFFFFull) return ctx.fail("attention: too many tasks");
-    if (a.splits > 1) {
-        const size_t accBytes = size_t(a.splits) * p.heads * p.count * p.dim * 4;
-        char* parts = static_cast<char*>(ctx.grow(SLOT_ATTN_PARTS, size_t(a.splits) * perSplit));
-        if (!parts) return false;
-        a.acc = reinterpret_cast<float*>(parts);
-        a.ml = reinterpret_cast<float2*>(parts + accBytes);
-    }
+    if (a.splits > 1 && !split_records(a)) return false;
     const bool d64 = p.dim == 64;
     if (!ctx.launch("attention_f32_tile_kernel", stream, [&] {
             if (d64) hipLaunchKernelGGL(attention_f32_tile_kernel<64>, dim3(unsigned(blocks)), dim3(256), 0, stream, a);
             else hipLaunchKernelGGL(attention_f32_tile_kernel<128>, dim3(unsigned(blocks)), dim3(256), 0, stream, a);
         }))
         return false;
-    if (a.splits == 1) return true;
-    const uint64_t mblocks = (p.count * p.heads + 3) / 4;
-    return ctx.launch("attention_f32_merge_kernel", stream, [&] {
-        if (d64) hipLaunchKernelGGL(attention_f32_merge_kernel<64>, dim3(unsigned(mblocks)), dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL(attention_f32_merge_kernel<128>, dim3(unsigned(mblocks)), dim3(256), 0, stream, a);
-    });
+    return a.splits == 1 || launch_merge(a, stream);
 }
 
 } // namespace

@@ -164,3 +164,61 @@ def test_tiled_fp32_unsplit_many_groups(gpu):
     say("tiled fp32 unsplit", cnt, H)
     got = gpu.attention(q, k, v, cnt, 0, H, KV, D, D)
     assert_f32_parity(ref, got[rows], "unsplit")
+
+
+# The narrow form (16 query rows of a kv head per workgroup, eight waves over
+# 16-key blocks), which small calls take, at the edges of its rows and blocks;
+# the last two have key ranges split over workgroups.
+@pytest.mark.parametrize("count,start,H,KV,D,window,stride", [
+    (1, 0, 1, 1, 64, 0, 64),         # one row, one key, seven waves without a block
+    (5, 11, 6, 2, 64, 0, 68),        # G = 3: a row group ends inside a token; 16 keys exactly
+    (17, 112, 12, 12, 64, 0, 64),    # 129 keys: one block past a step of the eight waves
+    (3, 1000, 32, 8, 128, 300, 128), # a window off the block boundary
+    (40, 3, 34, 2, 128, 20, 128),    # G = 17 > 16: a token over two row groups
+    (1, 2047, 32, 4, 128, 0, 128),
+    (33, 700, 10, 2, 64, 0, 64),
+])
+def test_narrow_fp32_shapes(gpu, count, start, H, KV, D, window, stride):
+    q = O.fill_normal((count, H, stride), 61, "q")
+    k = O.fill_normal((start + count, KV, D), 62, "k")
+    v = O.fill_normal((start + count, KV, D), 63, "v")
+    ref = O.attention(q, k, v, count, start, H, KV, D, stride, window)
+    say("narrow fp32", count, start, H, KV, D, window, stride)
+    got = gpu.attention(q, k, v, count, start, H, KV, D, stride, window)
+    assert_f32_parity(ref, got, f"narrow {count}/{start}/{D}/w{window}")
+
+
+@pytest.mark.parametrize("start", [100, 2000])   # one workgroup per row group; split
+def test_narrow_fp32_nonfinite_keys(gpu, start):
+    """a block's keys of -inf weigh nothing; a block's NaN keys reach every
+    output of their kv head and no other"""
+    count, H, KV, D = 2, 8, 2, 128
+    q = np.abs(O.fill_normal((count, H, D), 64, "q"))
+    k = O.fill_normal((start + count, KV, D), 65, "k")
+    v = O.fill_normal((start + count, KV, D), 66, "v")
+    ref = O.attention(q, np.ascontiguousarray(k[32:]), np.ascontiguousarray(v[32:]), count, start - 32, H, KV, D, D)
+    kinf = k.copy()
+    kinf[:32] = -np.inf
+    say("narrow fp32 -inf keys", start)
+    got = gpu.attention(q, kinf, v, count, start, H, KV, D, D)
+    assert_f32_parity(ref, got, f"narrow -inf keys {start}")
+    ref = O.attention(q, k, v, count, start, H, KV, D, D).reshape(count, H, D)
+    k[32:48, 0] = np.nan
+    say("narrow fp32 NaN keys", start)
+    got = np.asarray(gpu.attention(q, k, v, count, start, H, KV, D, D)).reshape(count, H, D)
+    assert np.isnan(got[:, :4]).all()
+    assert_f32_parity(ref[:, 4:], got[:, 4:], f"narrow NaN keys {start}")
+
+
+def test_tiled_fp32_split(gpu):
+    """256 tokens behind 2000 positions, 32q/8kv: the tiled form with its key
+    ranges split, sampled rows against the oracle"""
+    cnt, start, H, KV, D = 256, 2000, 32, 8, 128
+    q = O.fill_normal((cnt, H, D), 67, "q")
+    k = O.fill_normal((start + cnt, KV, D), 68, "k")
+    v = O.fill_normal((start + cnt, KV, D), 69, "v")
+    rows = sorted({0, 31, 32, 127, 128, 255} | set(range(5, 256, 29)))
+    ref = O.attention_strided(q.reshape(-1), k, v, cnt, start, H, KV, D, D, KV * D, D, rows=rows, nthreads=0)
+    say("tiled fp32 split", cnt, start)
+    got = gpu.attention(q, k, v, cnt, start, H, KV, D, D)
+    assert_f32_parity(ref, got[rows], "tiled split")
