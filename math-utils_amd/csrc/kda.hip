@@ -112,12 +112,21 @@ __device__ __forceinline__ void lower_block(int b, int& I, int& J) {
     so its own waves must cover each other's LDS reads and exps (four per SIMD
     at KD 128). In the two pairs of products at the end a wave has one
     16-column tile, whose column operand is read once and stays in registers,
-    and the rows of Tb and P come as 16-byte reads (k slot of step s: 16 M + 4 g
-    + s). Bound by its chain of short phases (a quarter of its cycles have an
+    and the rows of QKm, Tb and P come as 16-byte reads: their LDS columns are
+    permuted within each block of 16 (slot_of), so that a lane's four are its k
+    slots 16 M + 4 s + g of steps s = 0 .. 3.
+    The sums keep the order of four threads a row and 256 / KD runs of rows a
+    channel, whatever the number of threads: the in-chunk decays reach some
+    460, where fp32 steps are 2^-15, and the outputs follow their rounding (by
+    1e-4 of their root mean square at most, another order's by as much again).
+    Bound by its chain of short phases (a quarter of its cycles have an
     MFMA running): 2,048 workgroups (4,096 tokens, 32 heads of 128) 220 us, 235
     with eight waves, 305 with four and scalar operand reads.
 */
 template <int KD> constexpr int solve_threads() { return 8 * KD; }
+
+/* where column x of a 16-wide block of QKm, Tb and P sits in LDS (4 s + g at 4 g + s) */
+__device__ __forceinline__ int slot_of(int x) { return 4 * (x & 3) + (x >> 2); }
 
 template <int KD, bool F32>
 __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs a) {
@@ -153,14 +162,25 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
         float kx[PE], qx[PE];
         load_row<F32, PE>(p.k, (tr * p.keyHeads + kh) * KD + qq * PE, kx);
         load_row<F32, PE>(p.q, (tr * p.keyHeads + kh) * KD + qq * PE, qx);
+        // a quarter of a row is one chain over its QT threads, each taking the
+        // sum on where the one before it left off: after turn u it stands in
+        // the quarter's thread u
+        constexpr int QT = TR / 4;
         float kss = 0.0f, qss = 0.0f;
 #pragma unroll
-        for (int e = 0; e < PE; ++e) {
-            kss = fmaf(kx[e], kx[e], kss);
-            qss = fmaf(qx[e], qx[e], qss);
-        }
+        for (int u = 0; u < QT; ++u) {
+            kss = u ? __shfl_up(kss, 1, WAVE) : 0.0f;
+            qss = u ? __shfl_up(qss, 1, WAVE) : 0.0f;
 #pragma unroll
-        for (int o = 1; o < TR; o <<= 1) {
+            for (int e = 0; e < PE; ++e) {
+                kss = fmaf(kx[e], kx[e], kss);
+                qss = fmaf(qx[e], qx[e], qss);
+            }
+        }
+        kss = __shfl(kss, lane | (QT - 1), WAVE);
+        qss = __shfl(qss, lane | (QT - 1), WAVE);
+#pragma unroll
+        for (int o = QT; o < TR; o <<= 1) {
             kss += __shfl_xor(kss, o, WAVE);
             qss += __shfl_xor(qss, o, WAVE);
         }
@@ -232,22 +252,28 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
     __syncthreads();
 
     // ---- cumulative log2 decay of each channel down the chunk: the rows in
-    //      eight parts, each summed by its own thread, then offset ----
+    //      256 / KD parts, each summed by its own thread (four waves), then offset ----
     {
-        constexpr int PARTS = SOLVE_THREADS / KD, RPP = CH / PARTS;
+        constexpr int PARTS = 256 / KD, RPP = CH / PARTS;
         const int ch = tid % KD, part = tid / KD;
+        const bool mine = w < 4;   // uniform over the wave
         float col[RPP];
+        if (mine) {
 #pragma unroll
-        for (int r = 0; r < RPP; ++r) col[r] = gc[(part * RPP + r) * KS + ch];
+            for (int r = 0; r < RPP; ++r) col[r] = gc[(part * RPP + r) * KS + ch];
 #pragma unroll
-        for (int r = 1; r < RPP; ++r) col[r] += col[r - 1];
-        gc[(part * RPP + RPP - 1) * KS + ch] = col[RPP - 1];
+            for (int r = 1; r < RPP; ++r) col[r] += col[r - 1];
+            gc[(part * RPP + RPP - 1) * KS + ch] = col[RPP - 1];
+        }
         __syncthreads();
         float off = 0.0f;
-        for (int q2 = 0; q2 < part; ++q2) off += gc[((q2 + 1) * RPP - 1) * KS + ch];
+        if (mine)
+            for (int q2 = 0; q2 < part; ++q2) off += gc[((q2 + 1) * RPP - 1) * KS + ch];
         __syncthreads();
+        if (mine) {
 #pragma unroll
-        for (int r = 0; r < RPP; ++r) gc[(part * RPP + r) * KS + ch] = col[r] + off;
+            for (int r = 0; r < RPP; ++r) gc[(part * RPP + r) * KS + ch] = col[r] + off;
+        }
     }
     __syncthreads();
 
@@ -291,7 +317,7 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
             for (int rr = 0; rr < 4; ++rr) {
                 const int tt = r0 + 4 * g + rr;
                 Am[tt * CS + j] = (I != J || j < tt) ? bet[tt] * xa[rr] : 0.0f;
-                Qm[tt * CS + j] = (I != J || j <= tt) ? xq[rr] : 0.0f;
+                Qm[tt * CS + j0 + slot_of(c16)] = (I != J || j <= tt) ? xq[rr] : 0.0f;
             }
         } else {   // a diagonal block whose span is too wide to factorise
 #pragma unroll
@@ -305,7 +331,7 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
                     sq = fmaf(qn[t * KS + i], kj, sq);
                 }
                 Am[t * CS + j] = j < t ? bet[t] * sa : 0.0f;
-                Qm[t * CS + j] = j <= t ? sq : 0.0f;
+                Qm[t * CS + r0 + slot_of(c16)] = j <= t ? sq : 0.0f;
             }
         }
     }
@@ -350,10 +376,20 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
     }
     __syncthreads();
 
-    // ---- Tb = T diag(beta), in place ----
-    for (int idx = tid; idx < CH * CH; idx += SOLVE_THREADS) {
-        const int t = idx / CH, j = idx % CH;
-        if ((j >> 4) <= (t >> 4)) Tm[t * CS + j] *= bet[j];
+    // ---- Tb = T diag(beta), in place: a thread takes 16 columns of a row, which
+    //      it puts back permuted ----
+    for (int idx = tid; idx < CH * (CH / 16); idx += SOLVE_THREADS) {
+        const int t = idx / (CH / 16), j0 = 16 * (idx % (CH / 16));
+        if (j0 > t) continue;
+        floatx4 x[4], y[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[s] = *reinterpret_cast<const floatx4*>(&Tm[t * CS + j0 + 4 * s]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e][s] = x[s][e] * bet[j0 + 4 * s + e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *reinterpret_cast<floatx4*>(&Tm[t * CS + j0 + 4 * e]) = y[e];
     }
     __syncthreads();
 
@@ -365,10 +401,10 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
         for (int M = J; M <= I; ++M) {
             const floatx4 qm = *reinterpret_cast<const floatx4*>(&Qm[(16 * I + c16) * CS + 16 * M + 4 * g]);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) x = mfma4(qm[s], Tm[(16 * M + 4 * g + s) * CS + 16 * J + c16], x);
+            for (int s = 0; s < 4; ++s) x = mfma4(qm[s], Tm[(16 * M + 4 * s + g) * CS + 16 * J + slot_of(c16)], x);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) Am[(16 * I + 4 * g + r) * CS + 16 * J + c16] = x[r];
+        for (int r = 0; r < 4; ++r) Am[(16 * I + 4 * g + r) * CS + 16 * J + slot_of(c16)] = x[r];
     }
 
     // ---- the record: Kt and exp(gc_last) straight from kn, gc ----
@@ -414,11 +450,11 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
     // ---- -W = -Tb Kg and Qt = Qg - P Kg, computed transposed (key rows,
     //      token columns) so each lane's accumulator is one scan fragment ----
     {
-        float ak[4][4];   // Kg[16 M + 4 g + s][16 c + c16]
+        float ak[4][4];   // Kg[16 M + 4 s + g][16 c + c16]
 #pragma unroll
         for (int M = 0; M < 4; ++M)
 #pragma unroll
-            for (int s = 0; s < 4; ++s) ak[M][s] = kn[(16 * M + 4 * g + s) * KS + 16 * c + c16];
+            for (int s = 0; s < 4; ++s) ak[M][s] = kn[(16 * M + 4 * s + g) * KS + 16 * c + c16];
 #pragma unroll
         for (int I = 0; I < 4; ++I) {
             if (second != ((I == 0 || I == 3) ? 0 : 1)) continue;   // uniform
@@ -456,11 +492,11 @@ __global__ __launch_bounds__(solve_threads<KD>()) void kda_solve_kernel(KdaArgs 
         }
         __syncthreads();
         if (c < sw / 16) {
-            float bv[4][4];   // V[16 M + 4 g + s][16 c + c16]
+            float bv[4][4];   // V[16 M + 4 s + g][16 c + c16]
 #pragma unroll
             for (int M = 0; M < 4; ++M)
 #pragma unroll
-                for (int s = 0; s < 4; ++s) bv[M][s] = gc[(16 * M + 4 * g + s) * KS + 16 * c + c16];
+                for (int s = 0; s < 4; ++s) bv[M][s] = gc[(16 * M + 4 * s + g) * KS + 16 * c + c16];
             floatx4* blk = reinterpret_cast<floatx4*>(rUO + (c0 / 16 + c) * (2 * CH * 16));
 #pragma unroll
             for (int I = 0; I < 4; ++I) {

@@ -138,3 +138,61 @@ def test_raw_gates(gpu, safe):
     ro, rs = O.kda_rule(q, k, v, g, beta, state=s0, nthreads=0)
     assert_f32_parity(ro, host(out), f"out raw safe={safe}")
     assert_f32_parity(rs, host(state), f"state raw safe={safe}")
+
+
+def chunked_fp64(q, k, v, g, beta, order):
+    """the chunked form in float64 from in-chunk cumulative log2 decays that
+    are added in fp32 in `order`: 64 / order rows one after the other, then the
+    parts before them"""
+    S, H, KD = g.shape
+    out, state = np.zeros(v.shape), np.zeros((H, KD, v.shape[2]))
+    step = g * np.float32(1.4426950408889634)
+    norm = lambda x: x / np.sqrt((x.astype(np.float64) ** 2).sum(-1, keepdims=True) + 1e-6)
+    for c in range(0, S, 64):
+        n = min(64, S - c)
+        gc = np.zeros((n, H, KD), np.float32)
+        before, rows = np.zeros((H, KD), np.float32), 64 // order
+        for r0 in range(0, n, rows):
+            part = np.cumsum(step[c + r0:c + min(r0 + rows, n)], 0, dtype=np.float32)
+            gc[r0:r0 + rows] = part + before
+            before = before + part[-1]
+        for h in range(H):
+            G, Q, K, V = gc[:, h].astype(np.float64), norm(q[c:c + n, h]) / np.sqrt(KD), norm(k[c:c + n, h]), v[c:c + n, h]
+            b, S0 = beta[c:c + n, h].astype(np.float64)[:, None], state[h]
+            decay = np.exp2(np.minimum(G[:, None] - G[None], 0.0))
+            A = np.tril(b * np.einsum("ti,ji,tji->tj", K, K, decay), -1)
+            QK = np.tril(np.einsum("ti,ji,tji->tj", Q, K, decay))
+            U = np.linalg.solve(np.eye(n) + A, b * (V - (K * np.exp2(G)) @ S0))
+            out[c:c + n, h] = (Q * np.exp2(G)) @ S0 + QK @ U
+            state[h] = np.exp2(G[-1])[:, None] * S0 + (K * np.exp2(G[-1] - G)).T @ U
+    return out, state
+
+
+@pytest.mark.parametrize("kd", [128, 64])
+def test_order_of_the_decay_sums(gpu, kd):
+    """the in-chunk cumulative decays are added as 256 / kd runs of rows, in
+    that order and no other: a first decay of 2^-43281 in each chunk leaves
+    them 2^-8 apart, so that another order moves the outputs by 1e-4 and
+    more, where the products' rounding is held to the fp32 bar"""
+    import torch
+    S, H, vd = 150, 2, 32
+    q, k, v = (O.fill_normal((S, H, n), 81, name) for n, name in ((kd, "q"), (kd, "k"), (vd, "v")))
+    g = -O.fill_uniform((S, H, kd), 81, "g", 0.001, 0.1)
+    g[::64] = -30000.0
+    beta = O.fill_uniform((S, H), 81, "beta", 0.2, 0.9)
+    want, want_state = chunked_fp64(q, k, v, g, beta, 256 // kd)
+    other = chunked_fp64(q, k, v, g, beta, 8)[0]
+    assert np.abs(other - want).max() > 1e-4
+    state = dev_f32(np.zeros((H, kd, vd), np.float32))
+    out = torch.zeros((S, H, vd), dtype=torch.float32, device="cuda")
+    say("kda decay sums", dict(kd=kd))
+    gpu.kda_rule(dev_f32(q), dev_f32(k), dev_f32(v), dev_f32(g), dev_f32(beta), state, out)
+    assert_f32_parity(want, host(out), f"out kd={kd}")
+    assert_f32_parity(want_state, host(state), f"state kd={kd}")
+
+
+def test_long_sequence(gpu):
+    """64 chunks of 32 heads, more workgroups of the solve than the chip holds"""
+    ro, go, rs, gs = run_kda(gpu, 4096, 16, 32, 128, 128, 82, dtype="bf16")
+    assert_f32_parity(ro, go, "out 4096")
+    assert_f32_parity(rs, gs, "state 4096")
