@@ -35,7 +35,6 @@ enum ScratchSlot {
     SLOT_MIXER_KV,       // fp32 k and v projections of a prefill mixer before their epilogue
     SLOT_ATTN_PARTS,     // split records of the tiled fp32 attention
     SLOT_DELTA_SEG,      // segment maps and start states of the two-level delta-rule scan
-    SLOT_PREFILL_PARTS,  // key splits of a short prefill
     SLOT_COUNT
 };
 

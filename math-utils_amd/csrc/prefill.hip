@@ -1,6 +1,6 @@
 // prefill.hip - causal GQA prefill for gfx950.
 //
-// Two or three launches per call:
+// Two launches per call (three where prep does not convert the history):
 //   prefill_prep_kernel     attentionMixer's QK-RMSNorm -> RoPE -> KV append
 //                           (LocalModel.hpp:2608-2655) for the new tokens, in
 //                           fp32; writes the bf16 cache and the fp16 copies.
@@ -12,8 +12,6 @@
 //                           not run
 //   prefill_flash_kernel    flash attention on v_mfma_f32_32x32x16_f16 with
 //                           fp32 accumulation and an online softmax
-//   prefill_merge_kernel    (a short call behind a history) the key splits
-//                           combined
 //
 // Why fp16 operands: Q, K and P rounded to bf16 (8 significant bits) give
 // max-abs errors near 6e-3 on the 8k configuration; fp16 (11 bits) keeps
@@ -367,11 +365,6 @@ struct FlashArgs {
     uint32_t qStride, inType, half, fuseQ;
     uint32_t outputGate;   // out *= sigmoid(qraw[row + D + d]) (LocalModel.hpp:2660-2665)
     uint32_t* rangeFlag;   // set when a q element overflows fp16 (PrefillParams::rangeFlag)
-    // key splits (prefill_flash_kernel's SPLIT): each split's unnormalised
-    // rows [splits][count][heads][D] and its (max, sum) pairs
-    float* part;
-    float2* partMl;
-    uint32_t splits;
 };
 
 typedef __fp16 fp16x4 __attribute__((__vector_size__(4 * sizeof(__fp16))));
@@ -613,7 +606,7 @@ __device__ __forceinline__ void load_query(const FlashArgs& a, uint32_t tq, bool
     so the 4 rows x 64 bytes a 32-lane transposed read touches hit distinct
     banks.
 */
-template <int D, int WAVES, int STAGES, int BN, bool PP, bool SPLIT>
+template <int D, int WAVES, int STAGES, int BN, bool PP>
 __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_kernel(FlashArgs a) {
     static_assert(!PP || (WAVES == 8 && STAGES == 2 && BN == 128), "ping-pong: 8 waves, 2 stages, 128-key tiles");
     constexpr int BM = 32 * WAVES;
@@ -705,20 +698,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
     uint32_t kbeg = 0;
     if (a.window && a.start + q0 + 1 > a.window) kbeg = a.start + q0 + 1 - a.window;
     kbeg = kbeg / BN * BN;
-    uint32_t ntiles = (kend - kbeg + BN - 1) / BN;
-    // the row's (max, sum) of this split; lanes c and c + 32 hold one row
-    auto store_ml = [&](float mx, float sum) __attribute__((always_inline)) {
-        if (g == 0 && rowValid) a.partMl[(size_t(blockIdx.y) * a.count + tq) * a.heads + head] = float2{mx, sum};
-    };
-    if constexpr (SPLIT) {   // split blockIdx.y's share of the tiles
-        const uint32_t per = (ntiles + a.splits - 1) / a.splits, first = blockIdx.y * per;
-        if (first >= ntiles) {   // uniform, before any barrier
-            store_ml(-INFINITY, 0.0f);
-            return;
-        }
-        kbeg += first * BN;
-        ntiles = ntiles - first < per ? ntiles - first : per;
-    }
+    const uint32_t ntiles = (kend - kbeg + BN - 1) / BN;
 
     const _Float16* kbase = a.kh + size_t(kvh) * a.T * D;
     const _Float16* vbase = a.vh + size_t(kvh) * a.T * D;
@@ -1353,11 +1333,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
     }
 
     lsum += __shfl_xor(lsum, 32, WAVE);
-    if constexpr (SPLIT) store_ml(m, lsum);
-    float* const outRows = SPLIT ? a.part + size_t(blockIdx.y) * a.count * a.heads * D : a.out;
     bool direct = true;
     if constexpr (PP) {
-        if (SPLIT || (!a.outHi && !a.outputGate)) {
+        if (!a.outHi && !a.outputGate) {
             // The output rows leave through LDS. A lane's 16-byte pieces all
             // belong to its own row, so a store of them touches 32 cache lines
             // per instruction. Written to the wave's 16 KB of LDS (piece p of
@@ -1372,7 +1350,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
             const uint32_t wqe = q0 + 32 * wsc;
             const int wv = int(wsc);
             float* ob = reinterpret_cast<float*>(wv < 6 ? VP + wv * 8192 : K0 + (wv - 6) * 8192);
-            const float inv = wqe + uint32_t(ce) < a.count ? (SPLIT ? 1.0f : 1.0f / lsum) : 0.0f;
+            const float inv = wqe + uint32_t(ce) < a.count ? 1.0f / lsum : 0.0f;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -1389,13 +1367,13 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
                 const floatx4 val = *(lds_floatx4*)(ob + r * D + 4 * (p ^ (r & 15)));
                 const uint32_t row = wqe + uint32_t(r);
                 if (row < a.count)   // written once: nontemporal, so as not to displace K and V in L2
-                    __builtin_nontemporal_store(val, reinterpret_cast<floatx4*>(outRows + (size_t(row) * a.heads + head) * D + 4 * p));
+                    __builtin_nontemporal_store(val, reinterpret_cast<floatx4*>(a.out + (size_t(row) * a.heads + head) * D + 4 * p));
             }
         }
     }
     if (direct && rowValid) {
-        const float inv = SPLIT ? 1.0f : 1.0f / lsum;
-        float* dst = outRows + (size_t(tq) * a.heads + head) * D;
+        const float inv = 1.0f / lsum;
+        float* dst = a.out + (size_t(tq) * a.heads + head) * D;
         const size_t gateRow = (size_t(tq) * a.heads + head) * a.qStride + D;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
@@ -1404,14 +1382,14 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
                 floatx4 val;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) val[i] = o[dt][4 * r4 + i] * inv;
-                if (!SPLIT && a.outputGate) {   // sigmoidOf (LocalModel.hpp:1371) of the row's gate half
+                if (a.outputGate) {   // sigmoidOf (LocalModel.hpp:1371) of the row's gate half
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float gt = load_elem(a.qraw, gateRow + 32 * dt + 8 * r4 + 4 * g + i, int(a.inType));
                         val[i] *= 1.0f / (1.0f + expf(-gt));
                     }
                 }
-                if (!SPLIT && a.outHi) {   // the o projection's operand images, as split_a_kernel writes them
+                if (a.outHi) {   // the o projection's operand images, as split_a_kernel writes them
                     bf16x4 h, l;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -1425,59 +1403,6 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
                     *reinterpret_cast<floatx4*>(dst + 32 * dt + 8 * r4 + 4 * g) = val;
                 }
             }
-    }
-}
-
-/* the key splits of a row combined: out = sum_s 2^(m_s - M) o_s / sum_s
-   2^(m_s - M) l_s, through the output gate, as the flash kernel stores it.
-   D / 4 lanes a row, four columns each, every record requested at once. */
-template <int D>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(FlashArgs a) {
-    constexpr int LPR = D / 4, MAXS = 8;
-    const size_t rows = size_t(a.count) * a.heads;
-    const size_t row = size_t(blockIdx.x) * (256 / LPR) + threadIdx.x / LPR;
-    if (row >= rows) return;
-    const uint32_t d = 4 * (threadIdx.x % LPR);
-    float2 ml[MAXS];
-    floatx4 x[MAXS];
-#pragma unroll
-    for (int s = 0; s < MAXS; ++s) {
-        const bool in = uint32_t(s) < a.splits;
-        ml[s] = in ? a.partMl[s * rows + row] : float2{-INFINITY, 0.0f};
-        x[s] = in ? *reinterpret_cast<const floatx4*>(a.part + (s * rows + row) * D + d) : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    float M = -INFINITY, l = 0.0f;
-#pragma unroll
-    for (int s = 0; s < MAXS; ++s) M = fmaxf(M, ml[s].x);
-    floatx4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s = 0; s < MAXS; ++s) {
-        if (ml[s].x == -INFINITY) continue;   // no visible key there: its rows may be unwritten
-        const float f = __builtin_amdgcn_exp2f(ml[s].x - M);
-        l = fmaf(ml[s].y, f, l);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = fmaf(x[s][e], f, o[e]);
-    }
-    const float inv = 1.0f / l;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        o[e] *= inv;
-        if (a.outputGate) {
-            const float gt = load_elem(a.qraw, row * a.qStride + D + d + e, int(a.inType));
-            o[e] *= 1.0f / (1.0f + expf(-gt));
-        }
-    }
-    if (a.outHi) {
-        bf16x4 h, lo;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            h[e] = __bf16(o[e]);
-            lo[e] = __bf16(o[e] - float(h[e]));
-        }
-        *reinterpret_cast<bf16x4*>(a.outHi + row * D + d) = h;
-        *reinterpret_cast<bf16x4*>(a.outLo + row * D + d) = lo;
-    } else {
-        *reinterpret_cast<floatx4*>(a.out + row * D + d) = o;
     }
 }
 
@@ -1633,44 +1558,12 @@ bool launch_prefill(const PrefillParams& p, hipStream_t stream) {
     a.nQT = uint32_t((p.count + 32 * waves - 1) / (32 * waves));
     const uint64_t blocks = uint64_t(a.nQT) * p.heads;
     a.xcdRemap = (blocks % 8 == 0) ? 1u : 0u;
-    // a short call's query tiles leave CUs idle: the keys then split over the
-    // rest of them (at least three tiles each, or the merge launch, about 5 us,
-    // costs more than the 3 us a tile takes): 333 tokens after 1500, 32 heads:
-    // 64 workgroups of 15 tiles 48.7 us, 256 of 4 27.3 and the merge 6.5. Only
-    // behind a history: a row's fp16 probabilities round against its running
-    // maximum, so splits move its output by up to 3e-4, and a prompt from
-    // position 0 gives each row the same output whatever the call's length
-    const uint64_t seen = p.window && p.window + 32 * waves < T ? p.window + 32 * waves : T;
-    const uint32_t tiles = uint32_t((seen + 127) / 128);
-    uint64_t splits = blocks <= 128 ? 256 / blocks : 1;
-    if (splits > 8) splits = 8;
-    if (splits > tiles / 3) splits = tiles / 3;
-    if (p.start == 0) splits = 1;
-    if (splits > 1) {
-        const size_t rows = size_t(p.count) * p.heads;
-        a.part = static_cast<float*>(ctx.grow(SLOT_PREFILL_PARTS, splits * rows * (p.dim + 2) * sizeof(float)));
-        if (!a.part) return false;
-        a.partMl = reinterpret_cast<float2*>(a.part + splits * rows * p.dim);
-        a.splits = uint32_t(splits);
-        return ctx.launch("prefill_flash_kernel", stream, [&] {
-            const dim3 grid{unsigned(blocks), unsigned(splits)}, block{unsigned(64 * waves)};
-            if (p.dim == 128)
-                hipLaunchKernelGGL((prefill_flash_kernel<128, waves, 2, 128, true, true>), grid, block, 0, stream, a);
-            else
-                hipLaunchKernelGGL((prefill_flash_kernel<64, waves, 2, 128, false, true>), grid, block, 0, stream, a);
-        }) && ctx.launch("prefill_merge_kernel", stream, [&] {
-            const unsigned perBlock = unsigned(256 / (p.dim / 4));
-            const dim3 grid{unsigned((rows + perBlock - 1) / perBlock)};
-            if (p.dim == 128) hipLaunchKernelGGL(prefill_merge_kernel<128>, grid, dim3(256), 0, stream, a);
-            else hipLaunchKernelGGL(prefill_merge_kernel<64>, grid, dim3(256), 0, stream, a);
-        });
-    }
     return ctx.launch("prefill_flash_kernel", stream, [&] {
         const dim3 grid{unsigned(blocks)}, block{unsigned(64 * waves)};
         if (p.dim == 128)
-            hipLaunchKernelGGL((prefill_flash_kernel<128, waves, 2, 128, true, false>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((prefill_flash_kernel<128, waves, 2, 128, true>), grid, block, 0, stream, a);
         else
-            hipLaunchKernelGGL((prefill_flash_kernel<64, waves, 2, 128, false, false>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((prefill_flash_kernel<64, waves, 2, 128, false>), grid, block, 0, stream, a);
     });
 }
 

@@ -148,6 +148,5 @@ def test_rejects_mismatched_shapes(gpu):
 
 @pytest.mark.parametrize("kind,gate", [("bf16", False), ("q8", True)])
 def test_key_splits_behind_a_history(gpu, kind, gate):
-    """few rows behind 1500 positions: the attention's keys are split, and the merge writes the o projection's operand
-    images"""
+    """few rows behind 1500 positions: the attention writes the o projection's operand images"""
     run(gpu, kind, count=20, start=1500, gate=gate)

@@ -173,16 +173,66 @@ def test_output_gate_needs_wide_rows(gpu):
 
 
 @pytest.mark.parametrize("count,start,H,KV,D,window,gate,dtype", [
-    (1, 1151, 8, 2, 128, 0, False, "bf16"),     # 9 tiles in three splits, one row
-    (257, 640, 16, 8, 128, 0, False, "f32"),    # two query tiles, the second of one row; a split of it alone empty
-    (40, 2000, 4, 4, 128, 129, True, "bf16"),   # a window that leaves whole splits out of sight, the gate in the merge
+    (1, 1151, 8, 2, 128, 0, False, "bf16"),     # 9 full tiles, one row
+    (257, 640, 16, 8, 128, 0, False, "f32"),    # a query tile of one row
+    (40, 2000, 4, 4, 128, 129, True, "bf16"),   # a window of two tiles and a key, the gate
     (333, 1500, 8, 2, 64, 0, True, "bf16"), (20, 3000, 8, 8, 64, 1000, False, "f32"),
     (90, 1100, 6, 3, 128, 0, False, "bf16")])   # a grid that does not divide over the XCDs
 def test_key_splits_behind_a_history(gpu, count, start, H, KV, D, window, gate, dtype):
-    """a short call behind a history splits its keys over the idle CUs
-    (prefill_merge_kernel combines them), and its prep's extra workgroups
-    convert the history"""
+    """a short call behind a history, which its prep's extra workgroups convert"""
     ref, got, kn, v, kc, vcb, vb = run_case(gpu, count, start, H, KV, D, 70 + count, window=window, gate=gate,
                                             dtype=dtype, q_stride=2 * D if gate else None)
-    assert_bf16_parity(ref, got, f"splits {count} after {start}")
+    assert_bf16_parity(ref, got, f"{count} after {start}")
     assert np.abs(kc[:, start:start + count].transpose(1, 0, 2) - kn).max() <= np.abs(kn).max() * 2 ** -8
+
+
+@pytest.mark.parametrize("D,window,gate", [(128, 0, False), (64, 0, False), (128, 1000, True), (64, 700, True)])
+def test_rows_are_the_same_whatever_the_calls_length(gpu, D, window, gate):
+    """a token's output behind a history, bit for bit, in calls of 1, 20, 333 and
+    1100 tokens (one to five query tiles a head)"""
+    import torch
+    start, longest, H, KV = 1500, 1100, 32, 8
+    qs = 2 * D if gate else D
+    gen = torch.Generator(device="cuda").manual_seed(91)
+
+    def draw(*shape):
+        return torch.randn(shape, generator=gen, device="cuda").to(torch.bfloat16)
+
+    q, k, v = draw(longest, H, qs), draw(longest, KV, D), draw(longest, KV, D)
+    kc, vc = draw(KV, start + longest, D), draw(KV, start + longest, D)
+    gq, gk = dev_f32(gammas(D, 91, "q_norm")), dev_f32(gammas(D, 91, "k_norm"))
+    fr = dev_f32(O.rotary_frequencies(D, 1e6))
+
+    def rows(n):
+        out = torch.zeros((n, H, D), device="cuda")
+        say("prefill rows", dict(n=n, D=D, window=window, gate=gate))
+        gpu.prefill(q[:n], k[:n], v[:n], out, kc.clone(), vc.clone(), start, H, KV, D, q_stride=qs, q_norm=gq,
+                    k_norm=gk, freqs=fr, rotary_dims=D, window=window, output_gate=gate, check=True)
+        return host(out)
+
+    whole = rows(longest)
+    for n in (1, 20, 333):
+        assert np.array_equal(rows(n), whole[:n]), f"{n} tokens"
+
+
+@pytest.mark.parametrize("D,start,nan_at,window", [
+    (128, 1536, 1536, 0), (64, 1536, 1536, 0),      # the call's own key, the first of the last tile
+    (128, 1600, 1100, 501), (64, 1600, 1100, 501),  # the oldest key that the window leaves, cached
+])
+def test_a_nan_key_reaches_its_row(gpu, D, start, nan_at, window):
+    """one token whose visible keys hold one NaN at the edge of a key range: its
+    heads' outputs are NaN and the other kv head's are not"""
+    import torch
+    H, KV = 4, 2
+    q, k, v = (O.fill_normal((1, n, D), 92, name) for n, name in ((H, "q"), (KV, "k"), (KV, "v")))
+    kc, vc = (O.pack_bf16(O.fill_normal((KV, start + 1, D), 92, name)) for name in ("kc", "vc"))
+    kc, vc = dev_bf16(kc).view(KV, start + 1, D), dev_bf16(vc).view(KV, start + 1, D)
+    if nan_at == start:
+        k[0, 0, 3] = np.nan
+    else:
+        kc[0, nan_at, 3] = np.nan
+    out = torch.zeros((1, H, D), device="cuda")
+    say("prefill NaN key", dict(D=D, start=start, nan_at=nan_at, window=window))
+    gpu.prefill(dev_f32(q), dev_f32(k), dev_f32(v), out, kc, vc, start, H, KV, D, window=window)
+    got = host(out)
+    assert np.isnan(got[0, :2]).all() and np.isfinite(got[0, 2:]).all()
