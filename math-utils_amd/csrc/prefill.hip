@@ -43,6 +43,9 @@
 // rescaling is lazy (only when the max grows by more than 8 in log2 units).
 // D = 64 takes the single-phase loop: every wave computes S, the softmax and
 // P.V of each tile in turn, one barrier per tile.
+// Short calls, whose tiles of 256 query rows would leave CUs idle, take 64 rows
+// a workgroup and four waves for every 32 of them, with the same operations in
+// the same order (prefill_flash_shared_kernel).
 #include "context.hpp"
 #include "device.hpp"
 #include "kernels.hpp"
@@ -579,6 +582,41 @@ __device__ __forceinline__ void load_query(const FlashArgs& a, uint32_t tq, bool
         for (int db = 0; db < DB; ++db) {
             if (rowValid) qreg[db] = *reinterpret_cast<const half8*>(qrow + 16 * db + 8 * g);
             else qreg[db] = half8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
+}
+
+/* a lane's half of columns 32 dt .. + 31 of row tq of `head`, from the O^T
+   accumulator of d tile dt times inv, through the output gate */
+template <int D>
+__device__ __forceinline__ void store_columns(const FlashArgs& a, uint32_t tq, uint32_t head, int g, int dt,
+                                              const floatx16& o, float inv) {
+    const size_t at0 = (size_t(tq) * a.heads + head) * D + 32 * dt + 4 * g;
+    const size_t gate0 = (size_t(tq) * a.heads + head) * a.qStride + D + 32 * dt + 4 * g;
+#pragma unroll
+    for (int r4 = 0; r4 < 4; ++r4) {
+        floatx4 val;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) val[i] = o[4 * r4 + i] * inv;
+        if (a.outputGate) {   // sigmoidOf (LocalModel.hpp:1371) of the row's gate half
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gt = load_elem(a.qraw, gate0 + 8 * r4 + i, int(a.inType));
+                val[i] *= 1.0f / (1.0f + expf(-gt));
+            }
+        }
+        const size_t at = at0 + 8 * r4;
+        if (a.outHi) {   // the o projection's operand images, as split_a_kernel writes them
+            bf16x4 h, l;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                h[i] = __bf16(val[i]);
+                l[i] = __bf16(val[i] - float(h[i]));
+            }
+            *reinterpret_cast<bf16x4*>(a.outHi + at) = h;
+            *reinterpret_cast<bf16x4*>(a.outLo + at) = l;
+        } else {
+            *reinterpret_cast<floatx4*>(a.out + at) = val;
         }
     }
 }
@@ -1373,37 +1411,283 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 1) void prefill_flash_
     }
     if (direct && rowValid) {
         const float inv = 1.0f / lsum;
-        float* dst = a.out + (size_t(tq) * a.heads + head) * D;
-        const size_t gateRow = (size_t(tq) * a.heads + head) * a.qStride + D;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt) store_columns<D>(a, tq, head, g, dt, o[dt], inv);
+    }
+}
+
+/*
+    The flash kernel for short calls: 64 query rows of one head a workgroup, in
+    two groups of 32, and the four waves of a group share each 128-key tile of
+    it: wave kw scores keys 32 kw .. + 31, the group's row maxima, fp16
+    probabilities and row sums meet in LDS, and a wave accumulates its own 32
+    output columns (D = 64: two of the four waves) over all 128 keys. A row's
+    operations, their order and their roundings are those of
+    prefill_flash_kernel, so it comes out the same bits from either kernel and
+    does not depend on the length of its call.
+
+    The groups run one interval apart (a workgroup barrier ends each): group 0
+    has its products (P.V of tile j - 1, S of tile j) in interval 2j and the
+    softmax of tile j in 2j + 1, while group 1, whose waves share its SIMDs, has
+    the other. K and V are double-buffered. The softmax phase of tile j issues
+    the DMA of tile j + 1: group 0's of K, whose stage group 1 read two
+    intervals ago, to land in the same interval; group 1's of V, to land in the
+    next. Bound by the longer phase of each interval, the products (sixteen
+    dependent in two chains, 24 KB of operands a wave) or the softmax with its
+    DMA: at D = 128 1.35 us a tile, 1.6 with every CU busy, where the
+    eight-wave form takes 2.5 to 3.2 for 256 rows.
+*/
+template <int D>
+__global__ __launch_bounds__(512, 1) void prefill_flash_shared_kernel(FlashArgs a) {
+    constexpr int BN = 128, NKB = BN / 32, DB = D / 16, CPR = D / 8, RPB = WAVE / CPR;
+    constexpr int TILE = BN * D;                 // halfs per K or V tile
+    constexpr int PB = BN / RPB / 4;             // 1 KB DMA blocks per wave of a group and tile (K or V)
+    __shared__ __attribute__((aligned(16))) _Float16 Vs[2 * TILE];   // below 64 KB: V reads take immediate offsets
+    __shared__ __attribute__((aligned(16))) _Float16 Ks[2 * TILE];
+    __shared__ __attribute__((aligned(16))) half8 Ps[2][NKB][2][WAVE];   // P^T: [group][key block][half][lane]
+    __shared__ float2 Sums[2][NKB][WAVE];        // the lane's sums of its two 8-key runs of a key block
+    __shared__ float Max[2][NKB][32];            // row maxima of a key block
+
+    const uint32_t G = a.heads / a.kvHeads;
+    uint32_t lg = blockIdx.x;
+    if (a.xcdRemap) lg = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    const uint32_t kvh = lg / (G * a.nQT);
+    const uint32_t rest = lg % (G * a.nQT);
+    const uint32_t head = kvh * G + rest % G;
+    const uint32_t qt = a.nQT - 1 - rest / G;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, c = lane & 31;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6), rg = w >> 2, kw = w & 3;
+    // D = 64 has two column blocks: each group's on the SIMDs the other leaves idle
+    const int dt = D == 128 ? kw : kw & 1;
+    const bool pvWave = D == 128 || (kw >> 1) == rg;
+
+    const uint32_t q0 = qt * 64, wq0 = q0 + 32 * rg, tq = wq0 + c;
+    const bool rowValid = tq < a.count;
+    const uint32_t P = a.start + tq;
+    const uint32_t wLast = (wq0 + 31 < a.count ? wq0 + 31 : a.count - 1);
+    const uint32_t wPosFirst = a.start + wq0, wPosLast = a.start + wLast;
+    const uint32_t firstKey = (a.window && P + 1 > a.window) ? P + 1 - a.window : 0u;   // Kernels.hpp:142
+
+    const uint32_t tileLast = (q0 + 64 < a.count ? q0 + 64 : a.count) - 1;
+    const uint32_t kend = a.start + tileLast + 1;
+    uint32_t kbeg = 0;
+    if (a.window && a.start + q0 + 1 > a.window) kbeg = a.start + q0 + 1 - a.window;
+    kbeg = kbeg / BN * BN;
+    const uint32_t ntiles = (kend - kbeg + BN - 1) / BN;   // >= 1: count >= 1
+
+    const _Float16* kbase = a.kh + size_t(kvh) * a.T * D;
+    const _Float16* vbase = a.vh + size_t(kvh) * a.T * D;
+    // group 0 brings in K, group 1 V, laid out as prefill_flash_kernel's: blocks
+    // [n0, n1) of this wave's share of tile t into its stage; rows past the
+    // last key repeat it
+    const bool isK = rg == 0;
+    const _Float16* const src0 = isK ? kbase : vbase;
+    const uint32_t lds0 = lds_address(isK ? Ks : Vs) + uint32_t(kw * PB) * 1024;
+    auto issue = [&](uint32_t t, int n0, int n1) __attribute__((always_inline)) {
+        const uint32_t k0 = kbeg + t * BN;
+        const _Float16* src = src0 + size_t(k0) * D;
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                floatx4 val;
+        for (int n = n0; n < n1; ++n) {
+            const int i = (kw * PB + n) * RPB + lane / CPR, pos = lane % CPR;
+            uint32_t row = uint32_t(isK ? (i & ~31) + key_of_row(i & 31) : i);
+            if (k0 + row > a.T - 1) row = a.T - 1 - k0;
+            dma_block(src, 2 * (row * D + 8 * (pos ^ (isK ? kswz(i, D) : vswz(i, D)))), lds0 + (t & 1) * TILE * 2 + n * 1024);
+        }
+    };
+    issue(0, 0, PB);
+
+    half8 qreg[DB];
+    load_query<D>(a, tq, rowValid, head, g, qreg, nullptr, [] {});
+
+    // operand addresses as in prefill_flash_kernel
+    int kaddr[DB], vaddr;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) val[i] = o[dt][4 * r4 + i] * inv;
-                if (a.outputGate) {   // sigmoidOf (LocalModel.hpp:1371) of the row's gate half
+    for (int db = 0; db < DB; ++db) kaddr[db] = (32 * kw + c) * D + 8 * ((2 * db + g) ^ kswz(c, D));
+    {
+        const int q16 = lane & 15, half16 = (lane >> 4) & 1, rl = 16 * g + (q16 >> 2);
+        const int dbase = 32 * dt + 16 * half16 + 4 * (q16 & 3);
+        vaddr = rl * D + 8 * ((dbase >> 3) ^ vswz(rl, D)) + (dbase & 7);
+    }
+
+    // the tiles of which a row of the group sees a key: [jBegin, jEnd)
+    uint32_t jBegin = 0, jEnd = 0;
+    if (wq0 < a.count) {
+        if (a.window && uint64_t(wPosFirst) + 1 > a.window) jBegin = uint32_t(wPosFirst + 1 - a.window - kbeg) / BN;
+        jEnd = (wPosLast - kbeg) / BN + 1;
+    }
+
+    floatx16 o, s;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float gt = load_elem(a.qraw, gateRow + 32 * dt + 8 * r4 + 4 * g + i, int(a.inType));
-                        val[i] *= 1.0f / (1.0f + expf(-gt));
-                    }
+    for (int r = 0; r < 16; ++r) o[r] = 0.0f;
+    float m = -INFINITY, lsum = 0.0f, alpha = 1.0f;
+
+    // the product phase of tile j: O += P V of tile j - 1 (PV) and its row sums
+    // (HP), S of tile j (HS) and its maxima; two chains of products taken in
+    // turn, their operands read from LDS some eight reads ahead (the
+    // scheduling groups pin that order)
+    auto mphase = [&](uint32_t j, auto PV, auto HP, auto HS) __attribute__((always_inline)) {
+        constexpr bool pv = decltype(PV)::value, sc = decltype(HS)::value;
+        constexpr int N = 2 * NKB > DB ? 2 * NKB : DB;
+        const uint32_t k0 = kbeg + j * BN;
+        const _Float16* vs = Vs + ((j + 1) & 1) * TILE + vaddr;
+        const _Float16* ks = Ks + (j & 1) * TILE;
+        half8 vf[2 * NKB], pf[2 * NKB], kf[DB];
+        if constexpr (sc) {   // D = 128: S starts at -base, the running maximum (0 before the first key)
+            const float nb = D == 128 && m != -INFINITY ? -m : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[r] = nb;
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (pv && i < 2 * NKB) {
+                const _Float16* a0 = vs + (32 * (i / 2) + 8 * (i & 1)) * D;
+                vf[i] = read_tr16x2(a0, a0 + 4 * D);
+                pf[i] = Ps[rg][i / 2][i & 1][lane];
+            }
+            if (sc && i < DB) kf[i] = *reinterpret_cast<const half8*>(ks + kaddr[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (pv && i < 2 * NKB) o = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[i], pf[i], o, 0, 0, 0);
+            if (sc && i < DB) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[i], qreg[i], s, 0, 0, 0);
+        }
+        constexpr int BOTH = !pv || !sc ? 0 : (2 * NKB < DB ? 2 * NKB : DB), ONE = (pv ? 2 * NKB : (sc ? DB : 0)) - BOTH;
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+        for (int i = 0; i < BOTH; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < ONE; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, pv ? 3 : 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        if constexpr (decltype(HP)::value) {
+            float psum = 0.0f;
+            if constexpr (D == 128) {
+                float q[NKB];
+#pragma unroll
+                for (int kb = 0; kb < NKB; ++kb) {
+                    const float2 x = Sums[rg][kb][lane];
+                    q[kb] = x.x + x.y;
                 }
-                if (a.outHi) {   // the o projection's operand images, as split_a_kernel writes them
-                    bf16x4 h, l;
+                psum = (q[0] + q[1]) + (q[2] + q[3]);
+            } else {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        h[i] = __bf16(val[i]);
-                        l[i] = __bf16(val[i] - float(h[i]));
-                    }
-                    const size_t at = size_t(dst - a.out) + 32 * dt + 8 * r4 + 4 * g;
-                    *reinterpret_cast<bf16x4*>(a.outHi + at) = h;
-                    *reinterpret_cast<bf16x4*>(a.outLo + at) = l;
-                } else {
-                    *reinterpret_cast<floatx4*>(dst + 32 * dt + 8 * r4 + 4 * g) = val;
+                for (int kb = 0; kb < NKB; ++kb) {
+                    const float2 x = Sums[rg][kb][lane];
+                    psum += x.x;
+                    psum += x.y;
                 }
             }
+            lsum = lsum * alpha + psum;
+        }
+        if constexpr (sc) {
+            if ((k0 + BN - 1 > wPosFirst) || (a.window && uint64_t(k0) + a.window < uint64_t(wPosLast) + 1)) {
+                // keys outside [firstKey, P]: a -inf bit pattern from the sign, added
+                const int base = int(k0 + 32 * kw + 16 * g);
+                const int hi = int(P) - base;
+                const int lo = a.window ? int(firstKey) - base : -(1 << 30);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] += __int_as_float((((hi - r) | (r - lo)) >> 31) & int(0xFF800000u));
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+            if (g == 0) Max[rg][kw][c] = mx;
+        }
+    };
+    // the softmax phase of tile j (HS), and the DMA of tile j + 1
+    auto sphase = [&](uint32_t j, auto HS) __attribute__((always_inline)) {
+        const bool more = j + 1 < ntiles;
+        if (more) issue(j + 1, 0, PB / 2);
+        if constexpr (decltype(HS)::value) {
+            const float mx = fmaxf(fmaxf(Max[rg][0][c], Max[rg][1][c]), fmaxf(Max[rg][2][c], Max[rg][3][c]));
+            float shift;   // what the scores still have to lose
+            bool grow;
+            if constexpr (D == 128) {
+                const bool fresh = m == -INFINITY;
+                grow = fresh ? mx != -INFINITY : mx > 8.0f;
+                shift = grow ? mx : 0.0f;
+                alpha = fresh ? 0.0f : (grow ? __builtin_amdgcn_exp2f(-shift) : 1.0f);
+                if (grow) m = (fresh ? 0.0f : m) + shift;
+            } else {
+                grow = mx > m + 8.0f;
+                const float mn = grow ? mx : m;
+                alpha = grow ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;
+                shift = mn == -INFINITY ? 0.0f : mn;
+                m = mn;
+            }
+            float ps[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float e[8];
+                half8 pk;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    e[i] = __builtin_amdgcn_exp2f(s[8 * h + i] - shift);
+                    pk[i] = _Float16(e[i]);
+                }
+                ps[h] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+                Ps[rg][kw][h][lane] = pk;
+                if (h == 0 && more) issue(j + 1, PB / 2, PB);
+            }
+            Sums[rg][kw][lane] = float2{ps[0], ps[1]};
+            if (__any(grow)) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[r] *= alpha;
+            }
+        } else if (more) {
+            issue(j + 1, PB / 2, PB);
+        }
+    };
+
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    wait_vmcnt<0>();
+    lds_barrier();
+    // both phases of tile j and the two barriers: group 0's DMA lands in the
+    // interval that issued it, group 1's in the next
+    using Yes = std::true_type;
+    using No = std::false_type;
+    auto turn = [&](uint32_t j, auto RG, auto PV, auto HP, auto HS) __attribute__((always_inline)) {
+        mphase(j, PV, HP, HS);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if constexpr (decltype(RG)::value == 1) wait_vmcnt<0>();
+        lds_barrier();
+        if (j >= ntiles) return;
+        sphase(j, HS);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if constexpr (decltype(RG)::value == 0) wait_vmcnt<0>();
+        lds_barrier();
+    };
+    // the tiles before the group's, its first, its others, the products of its
+    // last, and the tiles after: ntiles turns and the products of one more
+    auto walk = [&](auto RG, auto PV) __attribute__((always_inline)) {
+        uint32_t j = 0;
+        for (; j < jBegin; ++j) turn(j, RG, No{}, No{}, No{});
+        if (j < jEnd) {
+            turn(j++, RG, No{}, No{}, Yes{});
+            for (; j < jEnd; ++j) turn(j, RG, PV, Yes{}, Yes{});
+            turn(j++, RG, PV, Yes{}, No{});
+        }
+        for (; j <= ntiles; ++j) turn(j, RG, No{}, No{}, No{});
+    };
+    using G0 = std::integral_constant<int, 0>;
+    using G1 = std::integral_constant<int, 1>;
+    if (rg == 0) {
+        if (pvWave) walk(G0{}, Yes{});
+        else walk(G0{}, No{});
+        lds_barrier();   // group 1's last products
+    } else {
+        lds_barrier();   // group 0's first products
+        if (pvWave) walk(G1{}, Yes{});
+        else walk(G1{}, No{});
     }
+    lsum += __shfl_xor(lsum, 32, WAVE);
+    if (rowValid && pvWave) store_columns<D>(a, tq, head, g, dt, o, 1.0f / lsum);
 }
 
 } // namespace
@@ -1552,18 +1836,28 @@ bool launch_prefill(const PrefillParams& p, hipStream_t stream) {
     a.half = p.freqs ? uint32_t(p.rotaryDims / 2) : 0u;
     a.outputGate = p.outputGate ? 1u : 0u;
     a.rangeFlag = p.rangeFlag;
-    // 8 waves of 32 query rows per workgroup, 128-key tiles: the ping-pong
-    // schedule for D = 128, the single-phase loop (two stages) for D = 64
-    constexpr int waves = 8;
-    a.nQT = uint32_t((p.count + 32 * waves - 1) / (32 * waves));
+    // 256 query rows a workgroup (D = 128: the ping-pong schedule; D = 64: the
+    // single-phase loop, two stages), or 64 of them in the form whose waves
+    // share a tile, where those workgroups fill the CUs at most once (D = 128)
+    // or twice (D = 64; 87 KB of LDS, one a CU all the same). With bf16 q, in
+    // us, 256 rows against 64: D = 128, 32 heads, 500 tokens after 1000 51.4
+    // and 39.3, 520 after 1000 (a second round) 50.3 and 52.8; D = 64 41.8 and
+    // 38.5, 1100 after 1000 (a third) 55.5 and 61.6
+    const uint64_t narrow = (p.count + 63) / 64 * p.heads;
+    const bool shared = narrow <= (p.dim == 128 ? 256 : 512);
+    a.nQT = uint32_t((p.count + (shared ? 63 : 255)) / (shared ? 64 : 256));
     const uint64_t blocks = uint64_t(a.nQT) * p.heads;
     a.xcdRemap = (blocks % 8 == 0) ? 1u : 0u;
     return ctx.launch("prefill_flash_kernel", stream, [&] {
-        const dim3 grid{unsigned(blocks)}, block{unsigned(64 * waves)};
-        if (p.dim == 128)
-            hipLaunchKernelGGL((prefill_flash_kernel<128, waves, 2, 128, true>), grid, block, 0, stream, a);
+        const dim3 grid{unsigned(blocks)}, block{512};
+        if (p.dim == 128 && shared)
+            hipLaunchKernelGGL((prefill_flash_shared_kernel<128>), grid, block, 0, stream, a);
+        else if (shared)
+            hipLaunchKernelGGL((prefill_flash_shared_kernel<64>), grid, block, 0, stream, a);
+        else if (p.dim == 128)
+            hipLaunchKernelGGL((prefill_flash_kernel<128, 8, 2, 128, true>), grid, block, 0, stream, a);
         else
-            hipLaunchKernelGGL((prefill_flash_kernel<64, waves, 2, 128, false>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((prefill_flash_kernel<64, 8, 2, 128, false>), grid, block, 0, stream, a);
     });
 }
 

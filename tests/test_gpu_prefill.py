@@ -186,10 +186,12 @@ def test_key_splits_behind_a_history(gpu, count, start, H, KV, D, window, gate, 
     assert np.abs(kc[:, start:start + count].transpose(1, 0, 2) - kn).max() <= np.abs(kn).max() * 2 ** -8
 
 
-@pytest.mark.parametrize("D,window,gate", [(128, 0, False), (64, 0, False), (128, 1000, True), (64, 700, True)])
+@pytest.mark.parametrize("D,window,gate", [(128, 0, False), (64, 0, False), (128, 1000, True), (64, 700, True),
+                                           (128, 40, False), (64, 129, False)])
 def test_rows_are_the_same_whatever_the_calls_length(gpu, D, window, gate):
-    """a token's output behind a history, bit for bit, in calls of 1, 20, 333 and
-    1100 tokens (one to five query tiles a head)"""
+    """a token's output behind a history, bit for bit, in calls of 1100 tokens
+    (256 query rows a workgroup) and of up to 333 (64, in two groups of 32:
+    one group, one row in the other, both, a second workgroup of one row)"""
     import torch
     start, longest, H, KV = 1500, 1100, 32, 8
     qs = 2 * D if gate else D
@@ -211,7 +213,7 @@ def test_rows_are_the_same_whatever_the_calls_length(gpu, D, window, gate):
         return host(out)
 
     whole = rows(longest)
-    for n in (1, 20, 333):
+    for n in (1, 20, 32, 33, 64, 65, 333):
         assert np.array_equal(rows(n), whole[:n]), f"{n} tokens"
 
 
