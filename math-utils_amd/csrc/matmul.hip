@@ -732,7 +732,7 @@ constexpr uint32_t CUS = 256;
    scales come in four at a time), 16-byte aligned rows, 32-bit byte offsets */
 bool dma_eligible(const GemvParams& p) {
     auto aligned = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) % 16) == 0; };
-    if (p.m < GEMM_MIN_M || p.k % (p.type >= 2 ? 4 * GD_BK : GD_BK) || !aligned(p.w) || !aligned(p.a) ||
+    if (p.m < GEMM_MIN_M || p.k == 0 || p.k % (p.type >= 2 ? 4 * GD_BK : GD_BK) || !aligned(p.w) || !aligned(p.a) ||
         (p.type >= 2 && !aligned(p.scales)))
         return false;
     const uint64_t rowBytes = uint64_t(p.k) / GD_BK * (p.type == 0 ? 128 : (p.type == 1 ? 64 : (p.type == 2 ? 32 : 16)));

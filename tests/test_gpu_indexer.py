@@ -193,3 +193,28 @@ def test_scores_of_values_that_are_not_finite(gpu, count):
             tol = 1e-4 * (np.abs(wt[t])[:, None] * (np.abs(q[t]) @ np.abs(p[:n]).T)).sum(0) + 1e-6
             tol = np.where(np.isfinite(tol), tol, 0.0)
             assert (np.abs(got[t, :n] - want)[~bad] <= tol[~bad]).all()
+
+
+@pytest.mark.parametrize("count", [1, 16])
+def test_rejects_an_empty_hidden_row(gpu, count):
+    """hidden = 0, whose projections have no terms, is refused whichever way the
+    rows of h would go (16 are enough for the matrix cores)"""
+    import ctypes as C
+
+    import aigpu
+    import torch
+    x = torch.zeros(64 * 64, dtype=torch.float32, device="cuda")
+    i = torch.zeros(1024, dtype=torch.int32, device="cuda")
+    f, n = C.c_void_p(x.data_ptr()), C.c_void_p(i.data_ptr())
+
+    def w(k_in, out):
+        return aigpu.AiGpuDenseWeight(codes=f, scales=None, type=aigpu.WEIGHT_TYPES["f32"], inDim=k_in, outDim=out, bias=None)
+
+    args = aigpu.AiGpuSelectKeys(h=f, qResid=f, idxK=w(0, 32), idxGate=w(0, 32), idxQB=w(8, 64), idxWeights=w(0, 2),
+                                 kNorm=f, kNormBias=None, ape=f, indexKeys=f, indexGates=f, poolKeys=f, selStart=n,
+                                 selCount=n, selKeys=n, scores=None, indexTail=1, count=count, startPos=0, hidden=0,
+                                 qRank=8, heads=2, dim=32, topK=8, pool=4, capacity=32,
+                                 stream=C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    say("select keys, hidden 0", dict(count=count))
+    assert gpu.lib().aigpu_select_keys(C.byref(args)) == 0
+    assert b"k must be positive" in gpu.lib().aigpu_last_error()
