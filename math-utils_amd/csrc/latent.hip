@@ -127,6 +127,13 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+/* 1 / the sum of a token's probabilities. An empty selection (no key at or
+   before the token) leaves the context at zero, as the mixer's job does; keys
+   whose scores are all -inf have no softmax: NaN, as a NaN among them gives. */
+__device__ __forceinline__ float context_scale(float l, bool empty) {
+    return l != 0.0f ? 1.0f / l : (empty ? 0.0f : __builtin_nanf(""));
+}
+
 /*
     Workgroup (token, 16 RT heads, key split), eight waves: online softmax over
     blocks of 32 keys. A block's latents come in by DMA (two 1 KB pieces a
@@ -278,13 +285,13 @@ __global__ __launch_bounds__(512, 2) void latent_attn_kernel(LatentArgs a) {
             }
 #pragma unroll
             for (int o = 1; o < TPR; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, WAVE));
-            const float mn = fmaxf(m, mx);   // the block's first key is live: finite for finite inputs
-            const float f = expf(m - mn);    // 0 on the first block
+            const float mn = fmaxf(m, mx), mz = mn == -INFINITY ? 0.0f : mn;   // all -inf so far: zeros (or NaN)
+            const float f = expf(m - mz);    // 0 on the first block
             m = mn;
             float ps = 0.0f;
 #pragma unroll
             for (int e = 0; e < KPT; ++e) {
-                const float pe = x[e] == -INFINITY ? 0.0f : expf(x[e] - mn);
+                const float pe = expf(x[e] - mz);
                 pr[sr * PS + sk + e] = pe;
                 ps += pe;
             }
@@ -330,9 +337,7 @@ __global__ __launch_bounds__(512, 2) void latent_attn_kernel(LatentArgs a) {
     for (int o = 1; o < TPR; o <<= 1) l += __shfl_xor(l, o, WAVE);
 
     if (a.splits == 1) {
-        // an empty selection (no key at or before the token) leaves the
-        // context at zero, as the mixer's job does (l = 0, acc = 0)
-        if (sk == 0) alpha[sr] = l > 0.0f ? 1.0f / l : (l == 0.0f ? 0.0f : l);
+        if (sk == 0) alpha[sr] = context_scale(l, n == 0);
         __syncthreads();
     }
     const size_t rec = size_t(C) + 4;
@@ -407,7 +412,7 @@ __global__ __launch_bounds__(256) void latent_unfold_kernel(LatentArgs a) {
             const float M = wave_max(mi);
             const float fi = mi != -INFINITY ? expf(mi - M) : 0.0f;
             const float L = wave_sum(li * fi);
-            const float inv = L > 0.0f ? 1.0f / L : (L == 0.0f ? 0.0f : L);   // every split empty: a zero context
+            const float inv = context_scale(L, p.selCount && p.selCount[t0 + t] == 0);
             floatx4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
             for (uint32_t i0 = odd; i0 < a.splits; i0 += 16) {   // eight records in flight
                 floatx4 x[8];

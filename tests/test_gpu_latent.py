@@ -114,3 +114,24 @@ def test_kv_b_off_16_byte_boundaries(gpu):
     gpu.latent_attention(dev_f32(q), dev_f32(latent), dw, out, start, 0.125)
     want = O.latent_attention(q, latent, wkv, start, heads, dn, dv, 0.125)
     assert np.abs(host(out) - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
+
+
+@pytest.mark.parametrize("start", [39, 63, 300])
+def test_scores_below_the_fp32_range_weigh_nothing(gpu, start):
+    """finite latents whose scores sum to -infinity: their probability is 0
+    wherever they stand (here the oldest 20 or 32 keys, a whole split or block),
+    and a token that sees no other is NaN, as exp(-inf - -inf) is"""
+    import torch
+    heads, dn, dv, C, far = 2, 8, 8, 64, 20 if start == 39 else 32
+    r = np.random.default_rng(13)
+    q = np.abs(r.standard_normal((1, heads, dn))).astype(np.float32)
+    wkv = np.abs(r.standard_normal((heads * (dn + dv), C))).astype(np.float32)
+    latent = (r.standard_normal((start + 1, C)) / 8).astype(np.float32)
+    want = O.latent_attention(q, latent[far:], wkv, start - far, heads, dn, dv, 0.125)
+    latent[:far] = -3e38
+    out = torch.zeros((1, heads, dv), dtype=torch.float32, device="cuda")
+    say("latent attention, scores of -inf", dict(start=start))
+    gpu.latent_attention(dev_f32(q), dev_f32(latent), dev_f32(wkv), out, start, 0.125)
+    assert np.abs(host(out) - want).max() <= 1e-5 * max(1.0, np.abs(want).max())
+    gpu.latent_attention(dev_f32(q), dev_f32(latent), dev_f32(wkv), out, far - 1, 0.125)
+    assert np.isnan(host(out)).all()
