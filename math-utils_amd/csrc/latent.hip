@@ -159,7 +159,7 @@ __global__ __launch_bounds__(512, 2) void latent_attn_kernel(LatentArgs a) {
     __shared__ __align__(16) float cb[2][KB * RS];
     __shared__ __align__(16) float sp[KP][16 * RT * PS];
     __shared__ __align__(16) float pr[16 * RT * PS];
-    __shared__ float alpha[16 * RT];
+    __shared__ __align__(16) float alpha[16 * RT];
 
     const LatentParams& p = a.p;
     const uint64_t t = blockIdx.x;
