@@ -486,7 +486,9 @@ AIGPU_ABI int aigpu_prefill_mixer(const AiGpuPrefillMixer* args);
 /*    best, plus the unfinished pool with indexTail. The result is the       */
 /*    selection aigpu_latent_attention takes. Among equal scores at the      */
 /*    boundary the lower pool is kept (the reference's nth_element leaves    */
-/*    that order unspecified). Device pointers throughout.                   */
+/*    that order unspecified). A score is fp32 work: within (dim + heads)    */
+/*    2^-24 of its terms' magnitudes, whatever range q and the pools span.   */
+/*    Device pointers throughout.                                            */
 /* ------------------------------------------------------------------------ */
 typedef struct AiGpuSelectKeys {
     const float* h;                 /* [count][hidden], latentAttentionMixer's input (the call, :3110) */

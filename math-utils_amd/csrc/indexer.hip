@@ -158,15 +158,27 @@ __global__ __launch_bounds__(256) void index_score_kernel(IndexArgs a, const flo
     for the whole launch; the workgroup's WT x WP waves take WT such token
     groups and share blocks of 64 pools in LDS (each wave 64 / WP of a block's
     pools). q and the pools are fp32: each row is scaled by a power of two to a
-    largest element in [2^10, 2^11) and split into two fp16 terms (22 bits),
-    and q.pool is three products, hi.hi + hi.lo + lo.hi, added in fp32 32
-    channels at a time. The terms left out are below 2^-22 of their product and
-    the sum is rounded four times instead of 128, so the dots carry less error
-    than the fp32 chain's (scores against float64, 1 to 500 tokens of 16 x 64
-    to 64 x 128 heads: 0.72 to 0.76 of it). relu commutes with the (positive) scales, so a lane
-    applies w headScale / scale_q once per head and dimScale / scale_pool once
-    per pool. A row that is not finite has no such split: its scores are formed
-    as index_score_kernel forms them.
+    largest element in [2^10, 2^11) and split into two fp16 terms, and q.pool is
+    three products, hi.hi + hi.lo + lo.hi, added in fp32 32 channels at a time.
+    The terms left out are below 2^-22 of their product and the sum is rounded
+    12 times instead of 128, so the dots carry less error than the fp32 chain's
+    (scores against float64, 1 to 500 tokens of 16 x 64 to 64 x 128 heads: 0.72
+    to 0.76 of it). relu commutes with the (positive) scales, so a lane applies
+    w headScale / scale_q once per head and dimScale / scale_pool once per pool.
+
+    An element under 2^-13 of its row's largest has fewer than 22 bits (2^-25 is
+    a half unit of the least fp16): 128 of them are off by at most 2^-6 of a
+    scaled dot. So each lane also adds |w| |dot| over its heads, and where that is
+    under its 2^12 sum |w|, the large channels of q meeting the small ones of the
+    pool, the 16 pools' scores are formed on the fp32 matrix cores; elsewhere
+    those 2^-6 are below 2^-18 of the score's terms, and all errors together
+    below 90 units of 2^-24 of them, where the fp32 chain's may reach 128 (rows
+    without such a mismatch have dots about their largest elements' product,
+    2^20 to 2^22). So are the scores of rows that are not finite or whose largest
+    element lies outside 2^+-50, and of head weights outside 2^-60 to 2^30, where
+    a scale times a weight could leave fp32's range. Errors of rows that span 2^0
+    to 2^+-26 are those of the fp32 chain or less; with every row spanning 2^+-26
+    the case below takes 1.0 ms (1.4 with index_score_kernel).
     Bound by the MFMAs (48 per 16 pools and wave, 8 KB of LDS reads):
     1024 tokens x 2,006 pools, 64 x 128: 1045 us with index_score_kernel (fp32
     FMA against LDS broadcasts), 120 us here; a decode step at 8,192 pools, the
@@ -190,6 +202,9 @@ __device__ __forceinline__ void split_half(const float (&x)[8], float scale, hal
     }
 }
 
+/* whether a row of largest element mx keeps its scale well inside fp32's range */
+__device__ __forceinline__ bool splittable(float mx) { return mx == 0.0f || (mx >= 0x1p-50f && mx <= 0x1p50f); }
+
 template <int HT, int WT, int WP>
 __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(IndexArgs a, const float* q, const float* w,
                                                                           const float* pools, float* scores) {
@@ -197,7 +212,7 @@ __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(Index
     constexpr int PIECES = IXM_BLOCK * IXM_DIM / 8 / THREADS;    // 8-channel pieces per thread and block
     constexpr int IMG = IXM_BLOCK * IXM_DIM;                     // halves of one image of a block
     __shared__ __align__(16) _Float16 img[2][2 * IMG];           // [buffer][hi, lo]
-    __shared__ float inv[2][IXM_BLOCK];                          // dimScale 2^-se of each pool, NaN: not finite
+    __shared__ float inv[2][IXM_BLOCK];                          // dimScale 2^-se of each pool (0: zeros), NaN: not split
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c16 = lane & 15;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wt = wv / WP, wp = wv % WP;
     const uint32_t nI = a.nI, Di = a.Di;
@@ -217,7 +232,7 @@ __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(Index
         const uint32_t t = t0 + i / HT, h = 16 * (i % HT) + c16;
         const bool live = t < a.count && h < nI;
         float x[IXM_KS][8], mx = 0.0f;
-        bool finite = true;
+        uint32_t bad = 0;
 #pragma unroll
         for (int s = 0; s < IXM_KS; ++s)
 #pragma unroll
@@ -229,7 +244,7 @@ __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(Index
                 for (int c = 0; c < 4; ++c) {
                     x[s][e + c] = v[c];
                     mx = fmaxf(mx, fabsf(v[c]));
-                    finite = finite && fabsf(v[c]) < INFINITY;
+                    bad |= fabsf(v[c]) < INFINITY ? 0u : 1u;
                 }
             }
         mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
@@ -238,12 +253,23 @@ __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(Index
         const float scale = ldexpf(1.0f, se);
 #pragma unroll
         for (int s = 0; s < IXM_KS; ++s) split_half(x[s], scale, ah[i][s], al[i][s]);
-        badQ = badQ || !finite;
-        const float wh = live ? w[size_t(t) * nI + h] * a.headScale * ldexpf(1.0f, -se) : 0.0f;
+        const float wr = live ? w[size_t(t) * nI + h] * a.headScale : 0.0f;
+        badQ = badQ || bad || !splittable(mx) || !(wr == 0.0f || (fabsf(wr) >= 0x1p-60f && fabsf(wr) <= 0x1p30f));
+        const float wh = mx == 0.0f ? 0.0f : wr * ldexpf(1.0f, -se);   // a row of zeros has no part in the scores
 #pragma unroll
         for (int r = 0; r < 4; ++r) coef[i][r] = __shfl(wh, 4 * g + r, WAVE);   // lane 4 g + r holds that row
     }
     badQ = __any(badQ);
+    float least[TPW];   // 2^12 sum |coef| of a token's heads in this lane
+#pragma unroll
+    for (int tk = 0; tk < TPW; ++tk) {
+        float v = 0.0f;
+#pragma unroll
+        for (int i = tk * HT; i < (tk + 1) * HT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v += fabsf(coef[i][r]);
+        least[tk] = v * 0x1p12f;
+    }
 
     // a block's pools: thread piece j is row (tid + THREADS j) / 16, channels 8 (tid % 16) ..
     float px[PIECES][8];
@@ -284,7 +310,7 @@ __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(Index
             const uint32_t at = row * IXM_DIM + 8 * (c ^ (row & 15));
             *reinterpret_cast<half8*>(&img[buf][at]) = hi;
             *reinterpret_cast<half8*>(&img[buf][IMG + at]) = lo;
-            if (c == 0) inv[buf][row] = bad ? __builtin_nanf("") : a.dimScale * ldexpf(1.0f, -se);
+            if (c == 0) inv[buf][row] = bad || !splittable(mx) ? __builtin_nanf("") : (mx == 0.0f ? 0.0f : a.dimScale * ldexpf(1.0f, -se));
         }
     };
 
@@ -320,36 +346,62 @@ __global__ __launch_bounds__(64 * WT * WP, 2) void index_score_mfma_kernel(Index
             }
             // relu, the head weights, and the sum over a token's heads: the
             // lane's four rows of each tile, then the four lane groups
-            float sum[TPW];
+            const uint32_t p = p0 + row;
+            bool again[TPW], any = false;   // the lane's scores to be formed from fp32 operands
 #pragma unroll
             for (int tk = 0; tk < TPW; ++tk) {
-                float v = 0.0f;
+                float v = 0.0f, size = 0.0f;
 #pragma unroll
                 for (int i = tk * HT; i < (tk + 1) * HT; ++i)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v = fmaf(coef[i][r], fmaxf(acc[i][r], 0.0f), v);
+                    for (int r = 0; r < 4; ++r) {
+                        v = fmaf(coef[i][r], fmaxf(acc[i][r], 0.0f), v);
+                        size = fmaf(fabsf(coef[i][r]), fabsf(acc[i][r]), size);
+                    }
                 v += __shfl_xor(v, 16, WAVE);
                 v += __shfl_xor(v, 32, WAVE);
-                sum[tk] = v * ip;
-            }
-            const uint32_t p = p0 + row;
-            const bool slow = badQ || !(ip == ip);
-#pragma unroll
-            for (int tk = 0; tk < TPW; ++tk) {
                 const uint32_t t = t0 + tk, complete = t < a.count ? (a.startPos + t + 1) / a.P : 0u;
-                if (g != 0 || p >= complete || sees_everything(a, complete)) continue;
-                float out = sum[tk];
-                if (slow) {   // a value that is not finite: the fp32 chain of index_score_kernel
-                    out = 0.0f;
-                    for (uint32_t h = 0; h < nI; ++h) {
-                        float d = 0.0f;
-                        for (uint32_t k = 0; k < Di; ++k)
-                            d = fmaf(q[(size_t(t) * nI + h) * Di + k], pools[size_t(p) * Di + k], d);
-                        const float logit = d * a.dimScale;
-                        out += w[size_t(t) * nI + h] * a.headScale * (logit > 0.0f ? logit : 0.0f);
+                const bool live = g == 0 && p < complete && !sees_everything(a, complete);
+                uint64_t small = __ballot(!(size >= least[tk]));   // a lane group whose dots are small
+                small |= small >> 32;
+                small |= small >> 16;
+                again[tk] = live && (badQ || !(ip == ip) || (ip != 0.0f && ((small >> c16) & 1)));
+                any = any || again[tk];
+                if (live && !again[tk]) scores[size_t(t) * a.maxPools + p] = v * ip;
+            }
+            if (__any(any)) {   // uniform over the wave; its 16 pools, on the fp32 matrix cores
+                floatx4 f[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) f[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+                const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (uint32_t d = 4 * g; d < IXM_DIM; d += 16) {   // k slot g of step e: channel d + e
+                    const floatx4 y = d < Di && p < most ? *reinterpret_cast<const floatx4*>(pools + size_t(p) * Di + d) : zero;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t t = t0 + i / HT, h = 16 * (i % HT) + c16;
+                        const floatx4 x = d < Di && t < a.count && h < nI
+                                              ? *reinterpret_cast<const floatx4*>(q + (size_t(t) * nI + h) * Di + d) : zero;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) f[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], f[i], 0, 0, 0);
                     }
                 }
-                scores[size_t(t) * a.maxPools + p] = out;
+#pragma unroll
+                for (int tk = 0; tk < TPW; ++tk) {
+                    const uint32_t t = t0 + tk;
+                    float v = 0.0f;
+#pragma unroll
+                    for (int i = tk * HT; i < (tk + 1) * HT; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const uint32_t h = 16 * (i % HT) + 4 * g + r;
+                            const float wh = t < a.count && h < nI ? w[size_t(t) * nI + h] * a.headScale : 0.0f;
+                            v = fmaf(wh, fmaxf(f[i][r] * a.dimScale, 0.0f), v);
+                        }
+                    v += __shfl_xor(v, 16, WAVE);
+                    v += __shfl_xor(v, 32, WAVE);
+                    if (again[tk]) scores[size_t(t) * a.maxPools + p] = v;
+                }
             }
         }
         if (p0 + stride < most) store(buf ^ 1);   // the other buffer's reads ended before the last barrier

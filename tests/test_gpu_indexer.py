@@ -218,3 +218,44 @@ def test_rejects_an_empty_hidden_row(gpu, count):
     say("select keys, hidden 0", dict(count=count))
     assert gpu.lib().aigpu_select_keys(C.byref(args)) == 0
     assert b"k must be positive" in gpu.lib().aigpu_last_error()
+
+
+@pytest.mark.parametrize("count", [2, 40])
+@pytest.mark.parametrize("spread,shift,w_shift", [(0, 0, 0), (8, 0, 0), (26, 0, 0), (13, 70, 0), (13, 100, 20), (0, -60, 0)])
+def test_scores_of_rows_of_wide_range(gpu, count, spread, shift, w_shift):
+    """large channels of q meet small channels of the pools: every score within
+    the bound of an fp32 chain of its dim + heads terms (2^-24 of the
+    magnitudes each), whatever 2^+-spread the channels and 2^shift the rows
+    span, and without an overflow that the score itself does not have"""
+    import torch
+    heads, dim, hidden, q_rank, start = 4, 128, 64, 8, 300
+    r = np.random.default_rng(15)
+    narrow = lambda *shape: (r.integers(64, 128, shape) * r.choice([-1, 1], shape) / 128).astype(np.float32)
+    span = np.exp2(r.integers(-spread, spread + 1, dim)).astype(np.float32)
+    # eight-bit mantissas and rows of a with a single 1: the projections are exact
+    wq = narrow(heads * dim, q_rank) * np.tile(span, heads)[:, None] * np.float32(2.0) ** shift
+    ww = narrow(heads, hidden) * np.float32(2.0) ** w_shift
+    w = {"k": narrow(dim, hidden), "gate": narrow(dim, hidden), "q": wq, "w": ww}
+    dev = {n: {"w": to_device(x), "kind": "f32", "out": x.shape[0], "in": x.shape[1], "scales": None}
+           for n, x in w.items()}
+    h, qr = np.zeros((count, hidden), np.float32), np.zeros((count, q_rank), np.float32)
+    h[:, 5] = 1.0
+    qr[np.arange(count), np.arange(count) % q_rank] = 1.0
+    cap = start + count + 1
+    pools = (r.standard_normal((cap + 1, dim)) / span * 2.0 ** -abs(shift) * (1 if shift >= 0 else 2.0 ** 120)).astype(np.float32)
+    keys, gates = (torch.zeros((cap, dim), dtype=torch.float32, device="cuda") for _ in range(2))
+    i32 = dict(dtype=torch.int32, device="cuda")
+    scores = torch.zeros((count, start + count), dtype=torch.float32, device="cuda")
+    say("select keys, wide rows", dict(count=count, spread=spread, shift=shift, w_shift=w_shift))
+    d_pools = dev_f32(pools)
+    gpu.select_keys(dev_f32(h), dev_f32(qr), dev, dev_f32(np.ones(dim)), None, dev_f32(np.zeros((1, dim))), keys, gates,
+                    d_pools, torch.zeros(count, **i32), torch.zeros(count, **i32), torch.zeros(count * 9, **i32), start,
+                    heads, dim, 8, 1, scores=scores)
+    got, p = host(scores).astype(np.float64), host(d_pools).astype(np.float64)
+    head = ww[:, 5].astype(np.float64) / np.sqrt(heads)
+    for t in range(count):
+        q = wq[:, t % q_rank].astype(np.float64).reshape(heads, dim)
+        dots = q @ p[:start].T / np.sqrt(dim)
+        size = np.abs(head) @ (np.abs(q) @ np.abs(p[:start]).T) / np.sqrt(dim)
+        err = np.abs(got[t, :start] - head @ np.maximum(dots, 0.0))
+        assert (err <= (dim + heads + 4) * 2.0 ** -24 * size).all(), f"token {t}: {np.nanmax(err / size):.3g} of the magnitudes"
