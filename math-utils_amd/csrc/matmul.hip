@@ -839,25 +839,25 @@ bool launch_dma(Context& ctx, const GemvParams* ps, int count, bool split, hipSt
             return false;
     }
     const dim3 grid(plan.tiles, plan.slices);
-    if (!ctx.launch("gemm_dma_kernel", stream, [&] {
-#define AIGPU_GD(T, BM, BN, WN)                             \
-    if (p.type == T && plan.bm == BM && plan.bn == BN)      \
-        hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WN>), grid, dim3(128 * WN), 0, stream, a)
-            AIGPU_GD(0, 128, 256, 4);
-            AIGPU_GD(0, 128, 128, 4);
-            AIGPU_GD(0, 64, 128, 2);
-            AIGPU_GD(1, 256, 256, 4);
-            AIGPU_GD(1, 128, 256, 4);
-            AIGPU_GD(1, 128, 128, 2);
-            AIGPU_GD(1, 64, 128, 2);
-            AIGPU_GD(2, 128, 256, 4);
-            AIGPU_GD(2, 128, 128, 2);
-            AIGPU_GD(2, 64, 128, 2);
-            AIGPU_GD(3, 128, 128, 2);
-            AIGPU_GD(3, 64, 128, 2);
+#define AIGPU_GD(T, BM, BN, WN)                                                                              \
+    if (p.type == T && plan.bm == BM && plan.bn == BN &&                                                     \
+        !ctx.launch("gemm_dma_kernel<" #T ", " #BM ", " #BN ">", stream, [&] {                               \
+            hipLaunchKernelGGL((gemm_dma_kernel<T, BM, BN, WN>), grid, dim3(128 * WN), 0, stream, a);        \
+        }))                                                                                                  \
+        return false
+    AIGPU_GD(0, 128, 256, 4);
+    AIGPU_GD(0, 128, 128, 4);
+    AIGPU_GD(0, 64, 128, 2);
+    AIGPU_GD(1, 256, 256, 4);
+    AIGPU_GD(1, 128, 256, 4);
+    AIGPU_GD(1, 128, 128, 2);
+    AIGPU_GD(1, 64, 128, 2);
+    AIGPU_GD(2, 128, 256, 4);
+    AIGPU_GD(2, 128, 128, 2);
+    AIGPU_GD(2, 64, 128, 2);
+    AIGPU_GD(3, 128, 128, 2);
+    AIGPU_GD(3, 64, 128, 2);
 #undef AIGPU_GD
-        }))
-        return false;
     if (plan.slices == 1) return true;
     const uint64_t quads = uint64_t(p.m) * plan.columns / 4;
     const unsigned rg = unsigned((quads + 255) / 256 < 65536 ? (quads + 255) / 256 : 65536);

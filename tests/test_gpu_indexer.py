@@ -259,3 +259,52 @@ def test_scores_of_rows_of_wide_range(gpu, count, spread, shift, w_shift):
         size = np.abs(head) @ (np.abs(q) @ np.abs(p[:start]).T) / np.sqrt(dim)
         err = np.abs(got[t, :start] - head @ np.maximum(dots, 0.0))
         assert (err <= (dim + heads + 4) * 2.0 ** -24 * size).all(), f"token {t}: {np.nanmax(err / size):.3g} of the magnitudes"
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8", "q4"])
+def test_projections_of_h_in_one_launch_of_k_slices(gpu, kind):
+    """k, the gates and w from 40 rows of h as three weights of one GEMM with K
+    slices: segments of 100, 100 and 20 columns in tiles of 128, each with its
+    bias, and a key cache that starts mid-way (run checks keys, gates and scores)"""
+    import torch
+    hidden, count, start, heads, dim = 2304, 40, 30, 20, 100
+    r = np.random.default_rng(17)
+    h = r.standard_normal((count, hidden)).astype(np.float32)
+    qr = r.standard_normal((count, 32)).astype(np.float32)
+    dev, dense, bias = {}, {}, {}
+    for name, (n, k) in {"k": (dim, hidden), "gate": (dim, hidden), "q": (heads * dim, 32), "w": (heads, hidden)}.items():
+        stored, scales, dense[name] = weight(n, k, "f32" if name == "q" else kind, 18, "seg" + name)
+        bias[name] = r.standard_normal(n).astype(np.float32)
+        dev[name] = {"w": to_device(stored), "kind": "f32" if name == "q" else kind, "out": n, "in": k,
+                     "scales": None if scales is None else dev_f32(scales), "bias": dev_f32(bias[name])}
+    cap = start + count + 1
+    keys, gates, pools = (torch.full((cap + 1, dim), 7.0, dtype=torch.float32, device="cuda") for _ in range(3))
+    i32 = dict(dtype=torch.int32, device="cuda")
+    scores = torch.zeros((count, start + count), dtype=torch.float32, device="cuda")
+    say("select keys, three weights in slices", dict(kind=kind))
+    gpu.profile_reset()
+    gpu.profile(True)
+    gpu.select_keys(dev_f32(h), dev_f32(qr), dev, dev_f32(np.ones(dim)), None, dev_f32(np.zeros((1, dim))), keys, gates,
+                    pools, torch.zeros(count, **i32), torch.zeros(count, **i32), torch.zeros(count * 5, **i32), start,
+                    heads, dim, 4, 1, scores=scores)
+    torch.cuda.synchronize()
+    gpu.profile(False)
+    assert gpu.profile_read("gemm_reduce_kernel")[1] == 1 and gpu.profile_read("gemm_dma_kernel")[1] == 2
+    h64, want = h.astype(np.float64), {}
+    for name in ("k", "gate", "w"):
+        want[name] = h64 @ dense[name].T.astype(np.float64) + bias[name]
+    tol = {n: 1e-5 * (np.abs(h64) @ np.abs(dense[n]).T.astype(np.float64)) + 1e-6 * (1 + np.abs(bias[n])) for n in want}
+    got = host(gates)
+    assert (np.abs(got[start:start + count] - want["gate"]) <= tol["gate"]).all()
+    assert (got[:start] == 7.0).all() and (got[start + count:] == 7.0).all()
+    k = want["k"]
+    mean, spread = k.mean(1, keepdims=True), np.sqrt(k.var(1, keepdims=True) + 1e-6)
+    got = host(keys)
+    assert (np.abs(got[start:start + count] - (k - mean) / spread) <= 4 * tol["k"].max() / spread + 1e-5).all()
+    q = (qr.astype(np.float64) @ dense["q"].T.astype(np.float64) + bias["q"]).reshape(count, heads, dim)
+    p64 = host(pools).astype(np.float64)
+    for t in range(count):
+        dots = q[t] @ p64[:start + t + 1].T / np.sqrt(dim)
+        size = (np.abs(want["w"][t]) + tol["w"][t])[:, None] / np.sqrt(heads) * (np.abs(q[t]) @ np.abs(p64[:start + t + 1]).T) / np.sqrt(dim)
+        ref = (want["w"][t][:, None] / np.sqrt(heads) * np.maximum(dots, 0)).sum(0)
+        assert (np.abs(host(scores)[t, :start + t + 1] - ref) <= 1e-4 * size.sum(0) + 1e-6).all(), f"token {t}"

@@ -72,8 +72,8 @@ def test_device_form(gpu, kind, m):
 
 @pytest.mark.parametrize("kind", ["bf16", "q8", "q4"])
 def test_split_k_for_few_tiles_and_long_k(gpu, kind):
-    """3 x 1 tiles against k = 7168: K is split into slices whose partial
-    tiles are added in order, then the bias and the residual"""
+    """five 64 x 128 tiles against k = 7168: K is split into 14 or 16 slices
+    whose partial tiles are added in order, then the bias and the residual"""
     import torch
     m, k, n = 300, 7168, 128
     a = O.fill_normal((m, k), 31, "a")
@@ -149,7 +149,8 @@ def test_rejects_quantised_k_not_multiple_of_32(gpu):
 
 @pytest.mark.parametrize("kind,k", [("f32", 100), ("bf16", 104), ("q8", 96), ("q4", 160)])
 def test_gemm_ragged_tiles(gpu, kind, k):
-    """the MFMA GEMM with m, n and k that do not fill its 128 x 128 x 32 tiles"""
+    """gemm_kernel (k that is not whole steps of the DMA GEMM) with m, n and k that
+    do not fill its 128 x 128 x 32 tiles"""
     import torch
     m, n = 131, 257
     a = O.fill_normal((m, k), 51, "a")
@@ -166,10 +167,10 @@ def test_gemm_ragged_tiles(gpu, kind, k):
 
 @pytest.mark.parametrize("k,accumulate", [(32, False), (96, True), (128, False)])
 def test_gemm_wide_tiles(gpu, k, accumulate):
-    """bf16 weights with enough 256 x 256 tiles for split_a_kernel and
-    gemm_dma_kernel (17 x 16 of them here, the last row and column of tiles
-    ragged; one, three and four K steps through its three-stage ring), bias,
-    and a residual add into a strided output"""
+    """bf16 weights against 4100 rows: one K step of 256 x 256 tiles, and three
+    and four of 128 x 128 (the ring of three stages not filled, filled once, and
+    refilled), the last row and column of tiles ragged, with the bias and a
+    residual add into a strided output"""
     import torch
     m, n, ld = 4100, 4000, 4008
     a = O.fill_normal((m, k), 61, "a")
@@ -188,8 +189,8 @@ def test_gemm_wide_tiles(gpu, k, accumulate):
 
 def test_one_row_against_a_wide_weight_takes_the_gemv(gpu):
     """a decode step's product against a wide weight (an LM head: one row of a,
-    65536 weight rows, 256 tiles of 256 x 256) runs on gemv_kernel: the DMA
-    GEMM's 256-row tiles would waste 255 of every 256 rows"""
+    65536 weight rows) runs on gemv_kernel: the DMA GEMM's tiles of 64 rows and
+    more would waste all but one of them"""
     import torch
     m, k, n = 1, 256, 65536
     a = O.fill_normal((m, k), 65, "a")
@@ -210,9 +211,8 @@ def test_one_row_against_a_wide_weight_takes_the_gemv(gpu):
 @pytest.mark.parametrize("kind", ["f32", "bf16", "q8", "q4"])
 @pytest.mark.parametrize("m,n,k", [(17, 130, 128), (65, 257, 640), (300, 1100, 384), (1030, 3000, 128), (2001, 4000, 256)])
 def test_gemm_dma_tiles(gpu, kind, m, n, k):
-    """gemm_dma_kernel at sizes from a part of its smallest tile to enough of its
-    largest, every tile row and column ragged: m, n one past or short of a
-    multiple, K of one group of four steps up, with and without K slices"""
+    """every encoding at the same sizes, m and n that leave tiles ragged, K of one
+    group of four steps up (test_gemm_dma_forms names each tile's shapes)"""
     import torch
     a = O.fill_normal((m, k), 71 + m, "a")
     w, scales, dense = weights(n, k, kind, 72 + n)
@@ -226,4 +226,58 @@ def test_gemm_dma_tiles(gpu, kind, m, n, k):
     err = np.abs(got[:, :n] - want)
     # the bar of this file, plus the residual add's own rounding
     assert np.all(err <= bound(a, dense) + 1e-6 * (1 + np.abs(base[:, :n]))), f"{kind}: max err {err.max()}"
+    np.testing.assert_array_equal(got[:, n:], base[:, n:])
+
+
+# every tile gemm_dma_kernel is built for, at the smallest shapes that take it
+# with the ring of three stages refilled twice (five K steps; twelve, three
+# groups of scales, for Q8 and Q4) and every edge ragged, and the forms with K
+# slices at shapes whose last slice is the shortest
+@pytest.mark.parametrize("kind,m,n,k,tile,sliced", [
+    ("f32", 17, 51, 160, (64, 128), False), ("f32", 17, 50, 480, (64, 128), True),
+    ("f32", 323, 5463, 160, (128, 128), False), ("f32", 2878, 50, 1568, (128, 128), True),
+    ("f32", 3617, 1043, 160, (128, 256), False), ("f32", 69, 5905, 2464, (128, 256), True),
+    ("bf16", 18, 59, 160, (64, 128), False), ("bf16", 17, 50, 832, (64, 128), True),
+    ("bf16", 4345, 395, 160, (128, 128), False), ("bf16", 65, 3037, 2336, (128, 128), True),
+    ("bf16", 2991, 1286, 160, (128, 256), False), ("bf16", 68, 5990, 4032, (128, 256), True),
+    ("bf16", 3929, 2085, 160, (256, 256), False), ("bf16", 1025, 3970, 3136, (256, 256), True),
+    ("q8", 19, 50, 384, (64, 128), False), ("q8", 17, 53, 1280, (64, 128), True),
+    ("q8", 4144, 402, 384, (128, 128), False), ("q8", 1396, 50, 4352, (128, 128), True),
+    ("q8", 4216, 899, 384, (128, 256), False), ("q8", 2765, 154, 2176, (128, 256), True),
+    ("q4", 18, 51, 384, (64, 128), False), ("q4", 23, 53, 1280, (64, 128), True),
+    ("q4", 3322, 515, 384, (128, 128), False), ("q4", 1370, 51, 4352, (128, 128), True)])
+def test_gemm_dma_forms(gpu, kind, m, n, k, tile, sliced):
+    """the form that the shape is here for has run, with bias and a residual add
+    into a strided output, against float64"""
+    import torch
+    r = np.random.default_rng(m + n)
+    a = r.standard_normal((m, k), dtype=np.float32)
+    src = r.standard_normal((n, k), dtype=np.float32)
+    if kind == "f32":
+        w, scales, dense = src, None, src
+    elif kind == "bf16":
+        w, scales = O.pack_bf16(src).reshape(n, k), None
+        dense = O.unpack_bf16(w).reshape(n, k)
+    else:
+        w, scales = quantise(src, kind)
+        dense = O.dequant(w, scales, kind)
+    bias = r.standard_normal(n, dtype=np.float32)
+    base = r.standard_normal((m, n + 3), dtype=np.float32)
+    out = dev_f32(base)
+    say("gemm dma form", dict(kind=kind, m=m, n=n, k=k, tile=tile, sliced=sliced))
+    gpu.profile_reset()
+    gpu.profile(True)
+    gpu.matmul(dev_f32(a), to_device(w), out[:, :n], kind, scales=None if scales is None else dev_f32(scales),
+               bias=dev_f32(bias), accumulate=True)
+    torch.cuda.synchronize()
+    gpu.profile(False)
+    form = f"gemm_dma_kernel<{('f32', 'bf16', 'q8', 'q4').index(kind)}, {tile[0]}, {tile[1]}>"
+    assert gpu.profile_read(form)[1] == 1, f"another tile than {form}"
+    assert gpu.profile_read("gemm_reduce_kernel")[1] == (1 if sliced else 0)
+    got = host(out)
+    a64, d64 = torch.from_numpy(a).cuda().double(), torch.from_numpy(np.ascontiguousarray(dense)).cuda().double()
+    want = (a64 @ d64.T).cpu().numpy() + bias + base[:, :n]
+    limit = 1e-5 * (a64.abs() @ d64.abs().T).cpu().numpy() + 1e-6 * (1 + np.abs(bias) + np.abs(base[:, :n]))
+    err = np.abs(got[:, :n] - want)
+    assert np.all(err <= limit), f"max err {err.max()}"
     np.testing.assert_array_equal(got[:, n:], base[:, n:])

@@ -109,15 +109,14 @@ def test_counts_and_history(gpu, count, start):
     (32, 16, 64, 32, True, 64, False, False), (2, 1, 64, None, False, 2048, False, True),
     (2, 1, 64, 32, True, 2048, True, False)])
 def test_fused_kv_projection(gpu, H, KV, D, rot, biases, hidden, gate, acc):
-    """8192 rows and 2 KV D = 2048 k and v columns make 256 tiles of 256 x 256:
-    k and v run as one DMA GEMM over both weights, then kv_epilogue_kernel. At
-    H D = 2048 the q projection takes the DMA GEMM too and its bf16 split of x
-    is reused; at H D = 1024 the pair splits x itself. At hidden = 2048 the o
-    projection has 256 such tiles too (here with 2 heads of 64, to keep the
-    oracle's projections short; k and v then take two launch_gemm_kv calls): the flash kernel then writes its bf16
-    operand images in place of fp32 rows (with the output gate applied first
-    when there is one), and the residual add rides on the GEMM. A window of 64
-    keeps the oracle's attention short."""
+    """every projection of 16 rows and more with whole K steps and aligned operands
+    takes the DMA GEMM: k and v run as one GEMM over both weights, then
+    kv_epilogue_kernel, and reuse the bf16 split of x that the q projection
+    left; the flash kernel writes its rows as the o projection's bf16 operand
+    images in place of fp32 rows (with the output gate applied first when there
+    is one), and the residual add rides on that GEMM. 8192 rows, in 256 x 256
+    tiles (hidden 64) and others; a window of 64 keeps the oracle's attention
+    short."""
     run(gpu, "bf16", count=8192, start=40, hidden=hidden, H=H, KV=KV, D=D, rot=rot, biases=biases, window=64,
         gate=gate, accumulate=acc)
 
@@ -150,3 +149,14 @@ def test_rejects_mismatched_shapes(gpu):
 def test_key_splits_behind_a_history(gpu, kind, gate):
     """few rows behind 1500 positions: the attention writes the o projection's operand images"""
     run(gpu, kind, count=20, start=1500, gate=gate)
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8", "q4"])
+def test_projections_in_k_slices(gpu, kind):
+    """few rows against hidden = 2304: every projection's K in slices, k and v (192
+    columns each, a tile and a half) as two weights of one launch"""
+    gpu.profile_reset()
+    gpu.profile(True)
+    run(gpu, kind, count=37, hidden=2304, H=6, KV=3, D=64, biases=True)
+    gpu.profile(False)
+    assert gpu.profile_read("gemm_reduce_kernel")[1] == 2   # q, and k with v (o has k = 384)
