@@ -178,11 +178,12 @@ __global__ __launch_bounds__(256) void index_score_kernel(IndexArgs a, const flo
     element lies outside 2^+-50, and of head weights outside 2^-60 to 2^30, where
     a scale times a weight could leave fp32's range. Errors of rows that span 2^0
     to 2^+-26 are those of the fp32 chain or less; with every row spanning 2^+-26
-    the case below takes 1.0 ms (1.4 with index_score_kernel).
+    the whole call of the case below takes 1.0 ms (1.4 with index_score_kernel,
+    0.25 with ordinary rows).
     Bound by the MFMAs (48 per 16 pools and wave, 8 KB of LDS reads):
     1024 tokens x 2,006 pools, 64 x 128: 1045 us with index_score_kernel (fp32
-    FMA against LDS broadcasts), 120 us here; a decode step at 8,192 pools, the
-    whole call: 91 and 86 us.
+    FMA against LDS broadcasts), 119 us here, 114 without the sums of |w| |dot|;
+    a decode step at 8,192 pools, the whole call: 77 and 72 us.
 */
 constexpr int IXM_DIM = 128, IXM_BLOCK = 64, IXM_KS = IXM_DIM / 32;
 

@@ -148,9 +148,9 @@ bool launch_gemv_presplit(const GemvParams& p, hipStream_t stream);
 // the k and v projections of the same rows (one GEMM over both weights where
 // the shapes allow), then the epilogue as its own kernel
 // fold: also write prep's cos/sin table (rope, may be null) and zero the
-// working copies' pad rows; *folded says whether that was done
+// working copies' pad rows, all that prep would do
 bool launch_gemm_kv_pair(const GemvParams& pk, const GemvParams& pv, const KvEpilogue& ek, const KvEpilogue& ev,
-                         bool aSplit, bool fold, float* rope, bool* folded, hipStream_t stream);
+                         bool aSplit, bool fold, float* rope, hipStream_t stream);
 
 // ---- attentionMixer for a prefill: projections, norm/RoPE/append, flash
 // attention, output gate, o projection ----

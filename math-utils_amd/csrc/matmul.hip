@@ -301,7 +301,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemvParams p, uint32_t kSlice
     row tile instead measured 20% slower). It is bound by the MFMA rate at the
     clock the chip holds: 1999 x 4096 -> 4096 in bf16, 128 x 256 tiles, 127 us
     (gemm_kernel, which splits a in registers and stores it to LDS behind two
-    barriers a step: 190); Q8 500 x 4096 -> 12288 137 us (217).
+    barriers a step: 190); Q8 500 x 4096 -> 12288, the whole call with the
+    split of a, 140 us (217; this kernel alone 151-155 under the tracer).
       BF16  up to 256 x 256 tiles
       F32   w in fp32 in LDS, split on its way into the operand registers
             (a third product, hi_a.lo_w)
@@ -595,11 +596,10 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a, uint32_t s
 
 /* The k and v projections' per-token work after one GEMM over both
    (kv[m][0 .. N1) k, [N1 .. 2 N1) v, fp32): the bias, then for k RMSNorm
-   (gamma) and rotate-half RoPE (freqs), and each row appended to its bf16
-   cache and to the flash kernel's fp16 copy, as gemm_kernel's k / v
-   epilogue does (the same operations in the same order per element; the
-   norm's sum of squares is reduced in another order). One workgroup per
-   token: the token's rotation angles float(pos) * freq go through sincosf
+   (gamma) and rotate-half RoPE (freqs) as norm_rope_row does them, and each
+   row appended to its bf16 cache and to the flash kernel's fp16 copy (the
+   rows the prep kernel would write). One workgroup per token: the token's
+   rotation angles float(pos) * freq go through sincosf
    once into LDS, then the four waves take its 2 * heads rows (k and v of
    each kv head) in turn, a row staged in LDS for the RoPE partner. A lane
    holds D / 64 consecutive elements. With rope set, the angles' cos and sin
@@ -980,9 +980,8 @@ bool launch_gemv_presplit(const GemvParams& p, hipStream_t stream) {
 }
 
 bool launch_gemm_kv_pair(const GemvParams& pk, const GemvParams& pv, const KvEpilogue& ek, const KvEpilogue& ev,
-                         bool aSplit, bool fold, float* rope, bool* folded, hipStream_t stream) {
+                         bool aSplit, bool fold, float* rope, hipStream_t stream) {
     Context& ctx = Context::instance();
-    *folded = false;
     if (pk.m == 0) return true;
     if (!kv_checks(ctx, pk, ek) || !kv_checks(ctx, pv, ev)) return false;
     if (pk.n != pv.n || pk.m != pv.m || pk.a != pv.a || ek.dim != ev.dim)
@@ -1005,13 +1004,10 @@ bool launch_gemm_kv_pair(const GemvParams& pk, const GemvParams& pv, const KvEpi
     uint4* padK = fold ? reinterpret_cast<uint4*>(static_cast<uint8_t*>(ek.work) + padAt) : nullptr;
     uint4* padV = fold ? reinterpret_cast<uint4*>(static_cast<uint8_t*>(ev.work) + padAt) : nullptr;
     const uint32_t pad16 = PREFILL_PAD_ROWS * ek.dim * 2 / 16;
-    if (!ctx.launch("kv_epilogue_kernel", stream, [&] {
-            hipLaunchKernelGGL(kv_epilogue_kernel, dim3(pk.m), dim3(256), 0, stream, kv, pk.bias, pv.bias, ek, ev,
-                               heads, fold ? rope : nullptr, padK, padV, pad16);
-        }))
-        return false;
-    *folded = fold;
-    return true;
+    return ctx.launch("kv_epilogue_kernel", stream, [&] {
+        hipLaunchKernelGGL(kv_epilogue_kernel, dim3(pk.m), dim3(256), 0, stream, kv, pk.bias, pv.bias, ek, ev, heads,
+                           fold ? rope : nullptr, padK, padV, pad16);
+    });
 }
 
 /* the shapes and alignments a k or v projection with its epilogue needs */
