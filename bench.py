@@ -5,8 +5,7 @@ with the reference's CPU path timed beside it.
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload prefill|decode|delta|small|published|bandwidth|gdn|kda|dense|gemm|mla|mixer|indexer|all]
 
 A step is one call of the hot path over one batch of synthetic, HBM-resident
-input. The headline workload (config.workload) is configs[2] of BASELINE.json,
-the Qwen3-8B-shaped causal GQA prefill at 8k (32 q / 8 kv heads, head_dim
+input. The headline workload (config.workload) is the Qwen3-8B-shaped causal GQA prefill at 8k (32 q / 8 kv heads, head_dim
 128, QK-RMSNorm + RoPE theta 1e6, bf16 in, fp32 accumulate): `value` is its
 whole-step TFLOP/s (norm/RoPE/append + flash attention) with the algorithmic
 count 2*D*Hq*S*(S+1). `configs` carries all five configurations in the same
@@ -46,18 +45,18 @@ sys.path.insert(0, os.path.join(ROOT, "math-utils_amd"))
 PEAK_MFMA_F16 = 2516.6      # TFLOP/s, dense bf16/fp16 MFMA (MI355X spec)
 PEAK_MFMA_F32 = 157.3       # TFLOP/s, fp32
 PEAK_HBM = 8000.0           # GB/s
-CPU_THREADS_CAP = 16        # the GPU box's CPU share for one GPU
+CPU_THREADS_CAP = 16        # a CPU baseline's threads: one GPU's share of its host
 
-# HBM bytes per launch of prefill_flash_kernel<128, 8, 2, 128, true> on
-# rocprofv3 FETCH_SIZE and WRITE_SIZE passes (`--calibrate-copy
+# HBM bytes per launch of prefill_flash_kernel<128, 8, 2, 128, true> at 8192
+# tokens, 32q/8kv heads: rocprofv3 FETCH_SIZE and WRITE_SIZE passes (`--calibrate-copy
 # --workload prefill`), each scaled by what the same counter reads for a
 # 1 GiB device copy (fetch x2.000, write x1.000): 182.1 MB read + 136.3 MB
 # written. Re-measure when the kernel changes.
 PREFILL_FLASH_TRAFFIC = 318.4e6
-# HBM bytes per launch of decode_attention_kernel<128> on configs[3], measured
+# HBM bytes per launch of decode_attention_kernel<128> on the ragged batch of 32, measured
 # the same way (`--workload decode`): 1,240.4 MB read + 5.2 MB written
 DECODE_ATTENTION_TRAFFIC = 1245.6e6
-# HBM bytes per step of the two-level delta scan on configs[4] (pass A, the
+# HBM bytes per step of the two-level delta scan at 16384 tokens (pass A, the
 # join and pass C together; `--workload delta`, the same scaling): pass A
 # 340.0 MB read + 29.7 MB written, the join 27.3 + 12.6 MB, pass C 402.9 +
 # 278.6 MB
@@ -85,7 +84,7 @@ def parse():
 # ------------------------------------------------------------ synthetic data
 class Xoshiro:
     """math::random::Random's randInt (Random.hpp:23-39, 67-86): only used to
-    draw configs[3]'s sequence lengths exactly as the configuration states."""
+    draw the ragged batch's sequence lengths as the reference would."""
     M = (1 << 64) - 1
 
     def __init__(self, seed):
@@ -182,7 +181,7 @@ def time_steps(step, steps, warmup, kernel, ramp_max=None):
 
 
 def parity(ref, got, max_abs_bar, rel_l2_bar=None, what=""):
-    """max-abs and rel-L2 (the north star's bars) and the reference's own
+    """max-abs and rel-L2 (the parity bars) and the reference's own
     maxAbs/rms (src/gpu-testing.cpp:85-95) of got against ref"""
     import numpy as np
     ref = np.asarray(ref, np.float64).reshape(-1)
@@ -272,7 +271,7 @@ def prefill_workload(args, cpu):
     step_ms, k_ms, launched_ms = time_steps(step, args.steps, args.warmup, "prefill_flash_kernel")
     aigpu.check_range()   # no fp16 range error in any timed call
     res = {
-        "workload": "configs[2] qwen3-8b causal GQA prefill S=8192 32q/8kv D=128 bf16, QK-norm+RoPE",
+        "workload": "qwen3-8b causal GQA prefill S=8192 32q/8kv D=128 bf16, QK-norm+RoPE",
         # bf16 in; the flash MFMAs take fp16 operands (3 more mantissa bits) and accumulate in fp32
         "dtype": "fp16",
         "value": flops / (step_ms * 1e-3) / 1e12, "unit": "TFLOP/s", "ms_per_step": step_ms,
@@ -294,7 +293,7 @@ def prefill_workload(args, cpu):
     wflops = 4.0 * D * H * sum(min(i + 1, W) for i in range(S))
     w_step, w_k, _ = time_steps(step_window, args.steps, args.warmup, "prefill_flash_kernel")
     aigpu.check_range()
-    res["window_4096"] = {"workload": "configs[2] shape with a sliding window of 4096 keys",
+    res["window_4096"] = {"workload": "the same shape with a sliding window of 4096 keys",
                           "value": wflops / (w_step * 1e-3) / 1e12, "unit": "TFLOP/s", "ms_per_step": w_step,
                           "kernel_ms": w_k, "kernel_frac": wflops / (w_k * 1e-3) / 1e12 / PEAK_MFMA_F16,
                           "flops_per_launch": wflops}
@@ -391,7 +390,7 @@ def decode_workload(args, cpu):
     step_ms, k_ms, launched_ms = time_steps(step, args.steps, args.warmup, "decode_attention_kernel")
     merge_ms, merge_n = aigpu.profile_read("decode_merge_kernel")   # pass 2 of time_steps
     res = {
-        "workload": "configs[3] qwen3-30b-a3b batched ragged GQA decode B=32 L~U[1k,32k] 32q/4kv D=128 bf16 KV",
+        "workload": "qwen3-30b-a3b batched ragged GQA decode B=32 L~U[1k,32k] 32q/4kv D=128 bf16 KV",
         "dtype": "bf16",
         "value": nbytes / (step_ms * 1e-3) / 1e9, "unit": "GB/s", "ms_per_step": step_ms,
         "step_frac": nbytes / (step_ms * 1e-3) / 1e9 / PEAK_HBM,
@@ -496,7 +495,7 @@ def delta_workload(args, cpu):
     step_ms, k_ms, launched_ms = time_steps(step, args.steps, args.warmup, scan_kernels)
     flops = S * HV * (7.0 * KD * VD + 4.0 * VD)
     res = {
-        "workload": "configs[4] qwen3-next gated delta rule S=16384 16qk/32v heads D=128 chunk 64 bf16 in, fp32 state",
+        "workload": "qwen3-next gated delta rule S=16384 16qk/32v heads D=128 chunk 64 bf16 in, fp32 state",
         # products on bf16 MFMA, each fp32 operand split into a bf16 high and
         # low part (three products), accumulated and kept in fp32
         "dtype": "bf16x3",
@@ -833,7 +832,7 @@ def mla_workload(args, cpu):
 
 
 def gdn_workload(args, cpu):
-    """the steps either side of the recurrence at configs[4]'s shapes: the fused
+    """the steps either side of the recurrence at Qwen3-Next's shapes: the fused
     qkvz de-interleave + causal conv (K 4) + SiLU, then the gated norm"""
     import numpy as np
     import torch
@@ -873,7 +872,7 @@ def gdn_workload(args, cpu):
     n_ms, n = aigpu.profile_read("gdn_gated_norm_kernel")
     n_ms = n_ms / n if n else float("nan")
     res = {
-        "workload": "configs[4] shapes: fused qkvz de-interleave + causal conv K=4 + SiLU (bf16 in/out), "
+        "workload": "qwen3-next shapes: fused qkvz de-interleave + causal conv K=4 + SiLU (bf16 in/out), "
                     "gated RMSNorm x SiLU(z) (fp32 x, bf16 z/out); S=16384 16k/32v heads D=128",
         "dtype": "bf16", "unit": "GB/s", "ms_per_step": step_ms,
         "value": (conv_bytes + norm_bytes) / (step_ms * 1e-3) / 1e9,
@@ -907,7 +906,7 @@ def gdn_workload(args, cpu):
 
 
 def cfg2_workload(args, cpu):
-    """configs[1]: Qwen3-0.6B decode, one token against 4096 cached positions
+    """Qwen3-0.6B decode, one token against 4096 cached positions
     (latency-bound: 16.8 MB of K and V)"""
     import numpy as np
     import torch
@@ -930,7 +929,7 @@ def cfg2_workload(args, cpu):
     step_ms, k_ms, launched_ms = time_steps(step, max(args.steps, 50), args.warmup, "decode_attention_kernel")
     merge_ms, merge_n = aigpu.profile_read("decode_merge_kernel")
     nbytes = 2.0 * (L + 1) * KV * D * 2
-    res = {"workload": "configs[1] qwen3-0.6b decode L=4096 16q/8kv D=128 bf16 KV, QK-norm+RoPE", "dtype": "bf16",
+    res = {"workload": "qwen3-0.6b decode L=4096 16q/8kv D=128 bf16 KV, QK-norm+RoPE", "dtype": "bf16",
            "unit": "GB/s", "value": nbytes / (step_ms * 1e-3) / 1e9, "ms_per_step": step_ms,
            "kernels_ms_per_step": launched_ms, "merge_kernel_ms": merge_ms / merge_n if merge_n else None,
            "roofline": {"kernel": "decode_attention_kernel", "bound": "hbm",
@@ -971,7 +970,7 @@ def cfg2_workload(args, cpu):
 
 
 def cfg1_workload(args, cpu):
-    """configs[0]: GPT-2-small MHA prefill, fp32, 128 tokens, through the
+    """GPT-2-small MHA prefill, fp32, 128 tokens, through the
     fp32 drop-in aigpu_attention_device (position-major KV, as kernels::attention)"""
     import numpy as np
     import torch
@@ -988,7 +987,7 @@ def cfg1_workload(args, cpu):
 
     step_ms, k_ms, launched_ms = time_steps(step, max(args.steps, 50), args.warmup, "attention_f32_narrow_kernel")
     flops = 4.0 * D * H * S * (S + 1) / 2
-    res = {"workload": "configs[0] gpt2-small MHA prefill fp32 S=128 12 heads D=64", "dtype": "f32",
+    res = {"workload": "gpt2-small MHA prefill fp32 S=128 12 heads D=64", "dtype": "f32",
            "unit": "TFLOP/s", "value": flops / (step_ms * 1e-3) / 1e12, "ms_per_step": step_ms,
            "roofline": {"kernel": "attention_f32_narrow_kernel", "bound": "fp32",
                         "achieved": flops / (k_ms * 1e-3) / 1e12, "peak": PEAK_MFMA_F32, "unit": "TFLOP/s",
@@ -1212,7 +1211,7 @@ def main():
                "latent_attention": "mla", "prefill_mixer": "mixer", "indexer": "indexer"}[name]
         if run(key):
             rows[name] = fn(args, cpu)
-    # the line's headline: configs[2] (prefill) when it ran, else the first that did
+    # the line's headline: the prefill when it ran, else the first that did
     order = ["cfg3", "cfg4", "cfg5", "cfg2", "cfg1"]
     head = next((configs[c] for c in order if c in configs), None)
     if head is None:

@@ -1,4 +1,4 @@
-"""Shared pieces of the parity tests: error metrics with the north-star
+"""Shared pieces of the parity tests: error metrics with their
 tolerances, and the seeded inputs of each configuration built with the
 restated reference RNG recipe (oracle.fill_*: Random(seed ^ fnv1a(name) +
 chunk*golden) per 2^14-element chunk, LocalModel.hpp:1555-1573)."""
@@ -6,7 +6,7 @@ import numpy as np
 
 from oracle import oracle as O
 
-# north-star tolerances
+# the parity bars
 BF16_MAX_ABS = 2e-3
 BF16_REL_L2 = 1e-3
 F32_MAX_ABS = 1e-5
